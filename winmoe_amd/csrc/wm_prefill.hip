@@ -517,68 +517,60 @@ int launch_prefill_route(const PrefillArgs& a, const int32_t* forced_ids, const 
 
 // One gate/up or down GEMM launch of format wt over the passes sel selects,
 // for passes of m pairs.
-template <int M> static int launch_q8(int nmat, int nsub, const PfGemm& g, int n_wg, hipStream_t s) {
-    if (nmat == 2) return launch_pf_gemm<1, 1, 2, Q8_0, M>(g, n_wg, s);     // gate and up in alternate stages
-    return nsub == 4 ? launch_pf_gemm<1, 2, 4, Q8_0, M>(g, n_wg, s) : launch_pf_gemm<1, 2, 2, Q8_0, M>(g, n_wg, s);
+template <int M> static int launch_q8(bool gateup, const PfGemm& g, int n_wg, hipStream_t s) {
+    return gateup ? launch_pf_gemm<1, 1, 2, Q8_0, M>(g, n_wg, s) : launch_pf_gemm<1, 2, 1, Q8_0, M>(g, n_wg, s);
 }
-static int launch_fmt(int m, int nmat, int nsub, int wt, const PfGemm& g, int n_wg, hipStream_t s) {
-    if (wt != Q8_0) return launch_pf_gemm_kq(m, nmat, nsub, wt, g, n_wg, s);
-    return m == 16 ? launch_q8<16>(nmat, nsub, g, n_wg, s) : launch_q8<32>(nmat, nsub, g, n_wg, s);
+static int launch_fmt(int m, bool gateup, int wt, const PfGemm& g, int n_wg, hipStream_t s) {
+    if (wt != Q8_0) return launch_pf_gemm_kq(m, gateup, wt, g, n_wg, s);
+    return m == 16 ? launch_q8<16>(gateup, g, n_wg, s) : launch_q8<32>(gateup, g, n_wg, s);
 }
 
-// Routed and shared passes in one launch when their formats agree, else in two.
-static int launch_split(int m, int nmat, int nsub, int wt_r, int wt_s, bool has_shared, PfGemm& g, int n_wg,
-                        hipStream_t s) {
-    if (!has_shared || wt_r == wt_s) {
-        g.sel = 0;
-        return launch_fmt(m, nmat, nsub, wt_r, g, n_wg, s);
-    }
-    g.sel = 1;
-    if (int rc = launch_fmt(m, nmat, nsub, wt_r, g, n_wg, s)) return rc;
+// Routed and shared passes in one launch when their formats and row lengths
+// agree, else in two.
+struct PfShape {
+    int wt, ncol;
+};
+static int launch_split(int m, bool gateup, PfShape r, PfShape sh, bool has_shared, PfGemm& g, int n_wg, hipStream_t s) {
+    const bool one = !has_shared || (r.wt == sh.wt && r.ncol == sh.ncol);
+    g.sel = one ? 0 : 1;
+    g.ncol = r.ncol;
+    g.rb = (int32_t)matrix_bytes(r.wt, 1, r.ncol);
+    if (int rc = launch_fmt(m, gateup, r.wt, g, n_wg, s)) return rc;
+    if (one) return 0;
     g.sel = 2;
-    return launch_fmt(m, nmat, nsub, wt_s, g, n_wg, s);
+    g.ncol = sh.ncol;
+    g.rb = (int32_t)matrix_bytes(sh.wt, 1, sh.ncol);
+    return launch_fmt(m, gateup, sh.wt, g, n_wg, s);
 }
 
 int launch_prefill_gateup(const PrefillArgs& a, hipStream_t s) {
     PfGemm g = {};
     g.w0 = a.gate; g.w1 = a.up; g.st0 = a.gstride; g.st1 = a.ustride;
     g.s0 = a.sh_gate; g.s1 = a.sh_up;
-    g.rb_r = matrix_bytes(a.gt, 1, a.H);
-    g.rb_s = a.has_shared ? matrix_bytes(a.sgt, 1, a.H) : g.rb_r;
-    g.mb_r = (int32_t)(g.rb_r * a.I);
-    g.mb_s = a.has_shared ? (int32_t)(g.rb_s * a.Is) : g.mb_r;
+    g.mb_r = (int32_t)matrix_bytes(a.gt, a.I, a.H);
+    g.mb_s = a.has_shared ? (int32_t)matrix_bytes(a.sgt, a.Is, a.H) : g.mb_r;
     g.a_hi = a.x16; g.a_lo = a.x16; g.a_ld = a.H; g.a_sc = nullptr; g.sc_ld = 0;
-    g.a_bytes = (int32_t)((int64_t)a.T * a.H * 2); g.sc_bytes = 0;
-    g.T = a.T; g.K = a.K; g.E = a.E; g.by_token = 1;
+    g.T = a.T; g.K = a.K;
+    g.rows_item = GM_ROWS;
     g.nrb_r = a.I / GM_ROWS; g.nrb_s = a.has_shared ? a.Is / GM_ROWS : 1;
-    g.ncol_r = g.ncol_s = a.H;
     g.recs = a.passes; g.npass = a.pass_count;
     g.o_hi = a.act_hi; g.o_lo = a.act_lo; g.o_sc = a.act_sc; g.o_ld = a.act_stride; g.osc_ld = a.act_stride / 128;
-    return launch_split(a.pass_m, 2, 1, a.gt, a.sgt, a.has_shared, g, a.n_wg, s);
+    return launch_split(a.pass_m, true, {a.gt, a.H}, {a.sgt, a.H}, a.has_shared, g, a.n_wg, s);
 }
 
 int launch_prefill_down(const PrefillArgs& a, hipStream_t s) {
     PfGemm g = {};
     g.w0 = a.down; g.w1 = a.down; g.st0 = g.st1 = a.dstride;
     g.s0 = g.s1 = a.sh_down;
-    g.rb_r = matrix_bytes(a.dt, 1, a.I);
-    g.rb_s = a.has_shared ? matrix_bytes(a.sdt, 1, a.Is) : g.rb_r;
-    g.mb_r = (int32_t)(g.rb_r * a.H); g.mb_s = (int32_t)(g.rb_s * a.H);
+    g.mb_r = (int32_t)matrix_bytes(a.dt, a.H, a.I);
+    g.mb_s = a.has_shared ? (int32_t)matrix_bytes(a.sdt, a.H, a.Is) : g.mb_r;
     g.a_hi = a.act_hi; g.a_lo = a.act_lo; g.a_ld = a.act_stride; g.a_sc = a.act_sc; g.sc_ld = a.act_stride / 128;
-    const int64_t pairs = (int64_t)a.T * a.K + (a.has_shared ? a.T : 0);
-    g.a_bytes = (int32_t)(pairs * a.act_stride * 2); g.sc_bytes = (int32_t)(pairs * (a.act_stride / 128) * 4);
-    g.T = a.T; g.K = a.K; g.E = a.E; g.by_token = 0;
-    g.ncol_r = a.I; g.ncol_s = a.has_shared ? a.Is : g.ncol_r;
+    g.T = a.T; g.K = a.K;
+    g.rows_item = a.H % 512 == 0 ? 512 : 256;
+    g.nrb_r = g.nrb_s = a.H / g.rows_item;
     g.recs = a.passes; g.npass = a.pass_count;
     g.y = a.y; g.y_ld = a.H;
-    // row groups of 4 blocks of 128 rows when H allows, else of 2 (H % 256
-    // == 0).  Q8_0 down takes groups of 2 whatever H: twice the items, so the
-    // last round of the persistent grid leaves less idle (C5: 1525 -> 1503 us
-    // per batch); for the K-quant down formats the groups of 4 measured
-    // faster (the Q4_K / Q6_K layer at 512 tokens: 1400 against 1404 us).
-    const int nsub = a.H % (4 * GM_ROWS) == 0 && a.dt != Q8_0 ? 4 : 2;
-    g.nrb_r = g.nrb_s = a.H / (nsub * GM_ROWS);
-    return launch_split(a.pass_m, 1, nsub, a.dt, a.sdt, a.has_shared, g, a.n_wg, s);
+    return launch_split(a.pass_m, false, {a.dt, a.I}, {a.sdt, a.Is}, a.has_shared, g, a.n_wg, s);
 }
 
 int launch_prefill_combine(const PrefillArgs& a, hipStream_t s) {
