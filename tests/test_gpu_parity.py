@@ -483,6 +483,38 @@ def test_prefill_router_kernels_agree(wm):
     assert L.prefill_status() == 0 and moved.prefill_status() == 0
 
 
+@pytest.mark.parametrize("T,E,H,K", [(1, 8, 256, 4), (15, 17, 512, 16), (16, 16, 1024, 16), (17, 96, 2048, 8),
+                                     (33, 40, 4096, 16), (360, 352, 256, 16), (545, 250, 1024, 16), (1025, 126, 256, 9)])
+def test_prefill_router_tiles(wm, orc, T, E, H, K):
+    """The matrix-core router at the edges of its tiles (16 x 16 below 128
+    tiles of 32 x 32, 32 x 32 from there; H of 2 to 32 chunks of 128): picks
+    and weights are those of the plain kernel (same layer, router 4 bytes past
+    a 16-byte boundary) bit for bit, with rows of subnormal, huge and equal
+    router values among the others."""
+    import torch
+    from winmoe_amd.moe import MoELayer
+    g = torch.Generator(device="cuda")
+    g.manual_seed(T * 131 + E)
+    R = 0.02 * torch.randn(E, H, generator=g, device="cuda")
+    R[E // 2] = R[E // 3]
+    R[0] *= 1e-37
+    R[E - 1] *= 1e30
+    X = torch.randn(T, H, generator=g, device="cuda").to(torch.bfloat16)
+    X[T // 2] *= 1e-30
+    buf = torch.zeros(E * H + 4, dtype=torch.float32, device="cuda")
+    shifted = buf[1:1 + E * H].view(E, H)
+    shifted.copy_(R)
+    I = 256
+    W = torch.zeros(E * I * (H // 32) * 34, dtype=torch.uint8, device="cuda")
+    ws = [MoELayer(H, I, E, K, r, W, W, W, (Q8_0, Q8_0, Q8_0), max_tokens=T) for r in (R, shifted)]
+    case(f"prefill router tiles T={T} E={E} H={H}")
+    for L in ws:
+        L.prefill(X)
+    (ia, wa), (ib, wb) = ([host(v) for v in L.prefill_routing(T)] for L in ws)
+    assert np.array_equal(ia, ib)
+    assert np.array_equal(wa.view(np.uint32), wb.view(np.uint32))
+
+
 def test_prefill_scales_and_narrow_shared(wm, orc):
     """Tokens whose magnitudes span 1e-6 .. 1e4 (one all zero, one with a
     single huge entry), a shared expert half as wide as the routed ones, an

@@ -5,7 +5,8 @@
 // (token, slot) pairs are grouped by expert and every expert's matrices are
 // streamed once for all of its tokens:
 //
-//   k_pf_router    reference-order fp32 logits of all tokens (tiles of 16
+//   k_pf_router_m  reference-order fp32 logits of all tokens on fp32 MFMA
+//   k_pf_router    the same for other widths and alignments (tiles of 16
 //                  tokens x 16 experts, each lane one of the 16 FMA chains of
 //                  4 x 4 (token, expert) pairs)
 //   k_pf_topk      one wave per token: K-pass arg-max + softmax
@@ -102,100 +103,162 @@ __global__ __launch_bounds__(256) void k_pf_router(const uint16_t* __restrict__ 
         }
 }
 
-// The same logits, for H a multiple of 128 and 16-byte aligned x rows and
-// router rows: tiles of 16 tokens x 32 experts, each thread the chain of
-// column residue l of 4 tokens x 8 experts (32 accumulators: 12 LDS reads per
-// 32 FMAs), the columns in chunks of 128 staged in LDS twice over: the loads
-// (16-byte vectors) of the next two chunks are in flight while the current
-// one is summed.  Every chain adds its columns in the same order as above, so the
-// logits are the same bit for bit.  LDS rows are 144 floats (16 mod 32 and
-// mod 64 banks) and the router row of local expert 8q + j is kept at row
-// q + 4j: the four expert groups of a wave (q = 0..3) read the same column of
-// rows q + 4j, 16 banks apart, with no conflict; rows stay 16-byte aligned
-// for the staging's 16-byte stores.
-constexpr int PQ_T = 16, PQ_E = 32, PQ_CH = 128, PQ_LD = PQ_CH + 16;
-WM_HD constexpr int pq_wrow(int e) { return (e >> 3) + 4 * (e & 7); }
-__global__ __launch_bounds__(256) void k_pf_router_v(const uint16_t* __restrict__ x, const float* __restrict__ W, int H,
+// The same logits on the matrix cores, for H a multiple of 128 and 16-byte
+// aligned x rows and router rows.  v_mfma_f32_16x16x1_4b_f32 adds one product
+// to each of 4 x 256 accumulators with a single rounding, the same bits as
+// fmaf (compared over normal and subnormal operands), so its 4 blocks are 4
+// of the 16 chains of a 16 x 16 (token, expert) tile: wave a runs the chains
+// a, a + 4, a + 8, a + 12, block b the chain of column residue a + 4 b, and
+// every chain adds its columns in the order above.  The xor tree's first two
+// levels add the blocks of a wave, its last two the four waves.
+//
+// A workgroup takes MT x ET such tiles.  The columns come in chunks of 128,
+// staged in LDS twice over with the loads of the next two chunks in flight.
+// A staging thread loads 4 columns (one for each wave) of 4 consecutive steps
+// of 16 columns and stores, per wave, the 4 steps as one 16-byte vector: the
+// operands of 4 MFMAs are then one 16-byte read.  LDS rows are 132 floats, so
+// the 16 rows of an operand read 16 different groups of 4 banks, and the
+// staging puts rows 8 apart next to each other for the same reason.
+//
+// Tiles of 32 x 32 read each row half as often as those of 16 x 16, which
+// spread a small batch over four times the workgroups: 32 x 32 from PQ_TILES
+// of them on.  Routing phase less a caller-routed one, us, 16 x 16 / 32 x 32:
+// 23 tokens, 512 experts, H 4096 (16 tiles of 32 x 32) 30.5 / 38.5; 100
+// tokens (64) 33.3 / 38.7; 1500 tokens, 96 experts (141) 66.0 / 51.4; 2000
+// tokens, 512 experts (1008) 255.6 / 149.1.  The kernel this replaced (16
+// FMA chains per thread on the vector units) took 49, 72 and 270 us alone
+// for 23, 512 and 2000 tokens, 512 experts.
+constexpr int PQ_CH = 128, PQ_LD = PQ_CH + 4, PQ_TILES = 128;
+typedef float f32x16 __attribute__((ext_vector_type(16)));
+template <int MT, int ET>
+__global__ __launch_bounds__(256) void k_pf_router_m(const uint16_t* __restrict__ x, const float* __restrict__ W, int H,
                                                      int T, int E, float* __restrict__ logits) {
-    __shared__ __attribute__((aligned(16))) float xs[2][PQ_T * PQ_LD];
-    __shared__ __attribute__((aligned(16))) float wsh[2][PQ_E * PQ_LD];
-    const int t0 = blockIdx.x * PQ_T, e0 = blockIdx.y * PQ_E;
-    const int tid = threadIdx.x, l = tid & 15, sb = tid >> 4, tq = sb >> 2, eq = sb & 3;
-    // staging: x row tid / 16, columns 8 (tid % 16) .. + 8 (one 16-byte load
-    // of bf16); W row tid / 8, columns 16 (tid % 8) .. + 16 (four)
-    const int xr = tid >> 4, xc = 8 * (tid & 15), wr = tid >> 3, wc = 16 * (tid & 7);
-    const bool xin = t0 + xr < T, win = e0 + wr < E;
-    const uint4* xsrc = (const uint4*)(x + (int64_t)(xin ? t0 + xr : 0) * H + xc);
-    const uint4* wsrc = (const uint4*)(W + (int64_t)(win ? e0 + wr : 0) * H + wc);
-    uint4 xv, wv[4], xv2, wv2[4];
-    auto gload = [&](int c0) {
-        const uint4 z = {0u, 0u, 0u, 0u};
-        xv = xin ? xsrc[c0 / 8] : z;
-#pragma unroll
-        for (int q = 0; q < 4; q++) wv[q] = win ? wsrc[c0 / 4 + q] : z;
+    constexpr int XN = (16 * MT * 8 + 255) / 256, WN = (16 * ET * 8 + 255) / 256;      // staging units per thread
+    __shared__ __attribute__((aligned(16))) float xs[2][16 * MT * PQ_LD];
+    __shared__ __attribute__((aligned(16))) float wsh[2][16 * ET * PQ_LD];
+    const int t0 = blockIdx.x * 16 * MT, e0 = blockIdx.y * 16 * ET;
+    const int tid = threadIdx.x, lane = tid & 63, a = __builtin_amdgcn_readfirstlane(tid >> 6), b = lane >> 4, i = lane & 15;
+    // staging unit u: steps 4 (u & 1) .. + 3 of the chunk, columns 4 bb .. + 3 of each step, of row `row`
+    auto unit = [&](int u, int& row, int& col, int& dst) __attribute__((always_inline)) {
+        const int kk = u & 1, bb = (u >> 1) & 3, r = u >> 3;
+        row = (r & ~15) + 8 * (r & 1) + ((r >> 1) & 7);
+        col = 64 * kk + 4 * bb;
+        dst = row * PQ_LD + 8 * bb + 4 * kk;
     };
-    auto gload2 = [&](int c0) {
-        const uint4 z = {0u, 0u, 0u, 0u};
-        xv2 = xin ? xsrc[c0 / 8] : z;
+    const uint16_t* xsrc[XN];
+    const float* wsrc[WN];
+    int xdst[XN], wdst[WN];
 #pragma unroll
-        for (int q = 0; q < 4; q++) wv2[q] = win ? wsrc[c0 / 4 + q] : z;
-    };
-    auto lstore = [&](int b) {
-        f32x4* xd = (f32x4*)&xs[b][xr * PQ_LD + xc];
-        xd[0] = (f32x4){bf16f((uint16_t)(xv.x & 0xFFFFu)), bf16f((uint16_t)(xv.x >> 16)),
-                        bf16f((uint16_t)(xv.y & 0xFFFFu)), bf16f((uint16_t)(xv.y >> 16))};
-        xd[1] = (f32x4){bf16f((uint16_t)(xv.z & 0xFFFFu)), bf16f((uint16_t)(xv.z >> 16)),
-                        bf16f((uint16_t)(xv.w & 0xFFFFu)), bf16f((uint16_t)(xv.w >> 16))};
-        f32x4* wd = (f32x4*)&wsh[b][pq_wrow(wr) * PQ_LD + wc];
-#pragma unroll
-        for (int q = 0; q < 4; q++) wd[q] = __builtin_bit_cast(f32x4, wv[q]);
-    };
-    float acc[4][8];
-#pragma unroll
-    for (int i = 0; i < 4; i++)
-#pragma unroll
-        for (int j = 0; j < 8; j++) acc[i][j] = 0.0f;
-    const int nch = H / PQ_CH;
-    gload(0);
-    lstore(0);
-    if (nch > 1) gload2(PQ_CH);
-    __syncthreads();
-    for (int c = 0; c < nch; c++) {
-        const int b = c & 1;
-        // chunk c + 1 is in flight in (xv2, wv2); chunk c + 2 goes out now
-        xv = xv2;
-#pragma unroll
-        for (int q = 0; q < 4; q++) wv[q] = wv2[q];
-        if (c + 2 < nch) gload2((c + 2) * PQ_CH);
-        const float* xb = &xs[b][(4 * tq) * PQ_LD + l];
-        const float* wb = &wsh[b][eq * PQ_LD + l];
-#pragma unroll 2
-        for (int st = 0; st < PQ_CH / 16; st++) {
-            float xq[4], wq[8];
-#pragma unroll
-            for (int i = 0; i < 4; i++) xq[i] = xb[i * PQ_LD + 16 * st];
-#pragma unroll
-            for (int j = 0; j < 8; j++) wq[j] = wb[4 * j * PQ_LD + 16 * st];
-#pragma unroll
-            for (int i = 0; i < 4; i++)
-#pragma unroll
-                for (int j = 0; j < 8; j++) acc[i][j] = fmaf(wq[j], xq[i], acc[i][j]);
-        }
-        // (the other buffer was last read before the previous barrier)
-        if (c + 1 < nch) lstore(b ^ 1);     // chunk c + 1
-        __syncthreads();
+    for (int q = 0; q < XN; q++) {
+        int row, col;
+        unit((tid + 256 * q) % (128 * MT), row, col, xdst[q]);
+        xsrc[q] = x + (int64_t)min(t0 + row, T - 1) * H + col;         // rows past the last repeat it (not stored)
     }
 #pragma unroll
-    for (int i = 0; i < 4; i++)
+    for (int q = 0; q < WN; q++) {
+        int row, col;
+        unit((tid + 256 * q) % (128 * ET), row, col, wdst[q]);
+        wsrc[q] = W + (int64_t)min(e0 + row, E - 1) * H + col;
+    }
+    struct Chunk {
+        uint2 x[XN][4];
+        f32x4 w[WN][4];
+    };
+    Chunk ca, cb;
+    auto gload = [&](Chunk& c, int c0) __attribute__((always_inline)) {
 #pragma unroll
-        for (int j = 0; j < 8; j++) {
-            float v = acc[i][j];
-            v += dpp_f32<DPP_ROR8>(v);
-            v += dpp_f32<DPP_ROR4>(v);
-            v += dpp_f32<DPP_ROR2>(v);
-            v += dpp_f32<DPP_ROR1>(v);
-            const int t = t0 + 4 * tq + i, e = e0 + 8 * eq + j;
-            if (l == 0 && t < T && e < E) logits[(int64_t)t * E + e] = v;
+        for (int q = 0; q < WN; q++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) c.w[q][j] = *(const f32x4*)(wsrc[q] + c0 + 16 * j);
+#pragma unroll
+        for (int q = 0; q < XN; q++)
+#pragma unroll
+            for (int j = 0; j < 4; j++) c.x[q][j] = *(const uint2*)(xsrc[q] + c0 + 16 * j);
+    };
+    auto lstore = [&](const Chunk& c, int buf) __attribute__((always_inline)) {
+#pragma unroll
+        for (int q = 0; q < WN; q++)
+            if (128 * ET >= 256 || tid < 128 * ET)
+#pragma unroll
+                for (int k = 0; k < 4; k++)
+                    *(f32x4*)&wsh[buf][wdst[q] + 32 * k] = (f32x4){c.w[q][0][k], c.w[q][1][k], c.w[q][2][k], c.w[q][3][k]};
+#pragma unroll
+        for (int q = 0; q < XN; q++)
+            if (128 * MT >= 256 || tid < 128 * MT)
+#pragma unroll
+                for (int k = 0; k < 4; k++) {
+                    f32x4 v;
+#pragma unroll
+                    for (int j = 0; j < 4; j++) {
+                        const uint32_t p = k < 2 ? c.x[q][j].x : c.x[q][j].y;
+                        v[j] = __builtin_bit_cast(float, (k & 1) ? p & 0xFFFF0000u : p << 16);
+                    }
+                    *(f32x4*)&xs[buf][xdst[q] + 32 * k] = v;
+                }
+    };
+    f32x16 acc[MT][ET];
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int e = 0; e < ET; e++) acc[m][e] = (f32x16)0.0f;
+    auto sums = [&](int buf) __attribute__((always_inline)) {
+        const float* xb = &xs[buf][i * PQ_LD + 32 * a + 8 * b];
+        const float* wb = &wsh[buf][i * PQ_LD + 32 * a + 8 * b];
+#pragma unroll
+        for (int kk = 0; kk < 2; kk++) {
+            f32x4 xv[MT], wv[ET];
+#pragma unroll
+            for (int m = 0; m < MT; m++) xv[m] = *(const f32x4*)(xb + 16 * m * PQ_LD + 4 * kk);
+#pragma unroll
+            for (int e = 0; e < ET; e++) wv[e] = *(const f32x4*)(wb + 16 * e * PQ_LD + 4 * kk);
+#pragma unroll
+            for (int j = 0; j < 4; j++)
+#pragma unroll
+                for (int m = 0; m < MT; m++)
+#pragma unroll
+                    for (int e = 0; e < ET; e++)
+                        acc[m][e] = __builtin_amdgcn_mfma_f32_16x16x1f32(xv[m][j], wv[e][j], acc[m][e], 0, 0, 0);
+        }
+    };
+    const int nch = H / PQ_CH;
+    gload(ca, 0);
+    if (nch > 1) gload(cb, PQ_CH);
+    lstore(ca, 0);
+    __syncthreads();
+    for (int c = 0; c < nch; c += 2) {
+        // chunk c is in buffer 0, c + 1 in flight in cb; c + 2 goes out now
+        // (a buffer was last read before the barrier ahead of its store)
+        if (c + 2 < nch) gload(ca, (c + 2) * PQ_CH);
+        sums(0);
+        if (c + 1 == nch) break;
+        lstore(cb, 1);
+        __syncthreads();
+        if (c + 3 < nch) gload(cb, (c + 3) * PQ_CH);
+        sums(1);
+        if (c + 2 < nch) lstore(ca, 0);
+        __syncthreads();
+    }
+    // s[a] = (chain a + chain a + 8) + (chain a + 4 + chain a + 12); the logit is (s[0] + s[2]) + (s[1] + s[3])
+    __syncthreads();
+    float(*red)[MT * ET * 256] = (float(*)[MT * ET * 256])&xs[0][0];
+    static_assert(4 * MT * ET * 256 <= 2 * 16 * MT * PQ_LD, "the partial sums take the x buffers' place");
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int e = 0; e < ET; e++)
+#pragma unroll
+            for (int r = 0; r < 4; r++)
+                red[a][(m * ET + e) * 256 + 64 * r + lane] =
+                    (acc[m][e][r] + acc[m][e][8 + r]) + (acc[m][e][4 + r] + acc[m][e][12 + r]);
+    __syncthreads();
+#pragma unroll
+    for (int m = 0; m < MT; m++)
+#pragma unroll
+        for (int e = 0; e < ET; e++) {
+            const int at = (m * ET + e) * 256 + tid;
+            const float v = (red[0][at] + red[2][at]) + (red[1][at] + red[3][at]);
+            const int t = t0 + 16 * m + 4 * b + (tid >> 6), ex = e0 + 16 * e + i;       // accumulator row 4 b + r, column i
+            if (t < T && ex < E) logits[(int64_t)t * E + ex] = v;
         }
 }
 
@@ -498,10 +561,15 @@ int launch_prefill_route(const PrefillArgs& a, const int32_t* forced_ids, const 
         hipLaunchKernelGGL(k_pf_forced, dim3((P + 255) / 256), dim3(256), 0, s, forced_ids, forced_w, P, a.E, a.ids, a.w,
                            a.hits, a.status);
     } else {
-        if (a.H % PQ_CH == 0 && ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.router & 15) == 0)
-            hipLaunchKernelGGL(k_pf_router_v, dim3((a.T + PQ_T - 1) / PQ_T, (a.E + PQ_E - 1) / PQ_E), dim3(256), 0, s,
-                               a.x, a.router, a.H, a.T, a.E, a.logits);
-        else
+        if (a.H % PQ_CH == 0 && ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.router & 15) == 0) {
+            const int64_t tiles = (int64_t)((a.T + 31) / 32) * ((a.E + 31) / 32);
+            if (tiles >= PQ_TILES)
+                hipLaunchKernelGGL((k_pf_router_m<2, 2>), dim3((a.T + 31) / 32, (a.E + 31) / 32), dim3(256), 0, s, a.x,
+                                   a.router, a.H, a.T, a.E, a.logits);
+            else
+                hipLaunchKernelGGL((k_pf_router_m<1, 1>), dim3((a.T + 15) / 16, (a.E + 15) / 16), dim3(256), 0, s, a.x,
+                                   a.router, a.H, a.T, a.E, a.logits);
+        } else
             hipLaunchKernelGGL(k_pf_router, dim3((a.T + PR_T - 1) / PR_T, (a.E + PR_E - 1) / PR_E), dim3(256), 0, s, a.x,
                                a.router, a.H, a.T, a.E, a.logits);
         hipLaunchKernelGGL(k_pf_topk, dim3((a.T + WAVES - 1) / WAVES), dim3(256), 0, s, a.logits, a.T, a.E, a.K, a.ids,
