@@ -546,6 +546,37 @@ def test_prefill_scales_and_narrow_shared(wm, orc):
     assert sl.layer.prefill_status() == 0
 
 
+@pytest.mark.parametrize("H,I,types,sh_inter", [
+    (1024, 256, (Q8_0, Q8_0, Q8_0), 0), (4096, 1024, (Q8_0, Q8_0, Q8_0), 256), (2048, 512, (Q4_K, Q4_K, Q6_K), 512),
+    (4096, 256, (Q3_K, Q3_K, Q4_K), 1024), (512, 2048, (Q4_K, Q4_K, Q6_K), 256), (256, 1024, (Q6_K, Q6_K, Q2_K), 256)])
+def test_prefill_batch_split(wm, orc, H, I, types, sh_inter):
+    """A token's output does not depend on its batch, bit for bit, where the
+    batch's size picks the down items (128, 256 or 512 rows), the pass size
+    and the rounds of the grid, and the row lengths the waves of a workgroup
+    (1 to 8 slices) and whether routed and shared passes share a launch; one
+    token against the oracle."""
+    from winmoe_amd import synth
+    E, K, T = 48, 6, 1100
+    cfg = synth.LayerConfig(f"pf_split_{H}_{I}_{types[0]}", E=E, K=K, H=H, I=I, types=types,
+                            shared_types=(Q8_0,) * 3 if sh_inter else None, shared_inter=sh_inter,
+                            shared_gate_inp=bool(sh_inter), tokens=1, routing="zipf", x_dtype="bf16", seed=5)
+    sl = synth.build_layer(cfg, max_tokens=T)
+    X = synth.make_hidden(cfg, tokens=T)
+    rng = np.random.default_rng(H + I)
+    ids = np.stack([rng.choice(E, K, replace=False) for _ in range(T)]).astype(np.int32)
+    w = rng.random((T, K)).astype(np.float32)
+    case(f"prefill split H={H} I={I} types={types} shared={sh_inter}")
+    whole = host(sl.layer.prefill_forced(X, dev(ids), dev(w)))
+    assert np.isfinite(whole).all()
+    for n in (1, 3, 40, 333):
+        case(f"prefill split n={n}")
+        part = host(sl.layer.prefill_forced(X[:n].contiguous(), dev(ids[:n]), dev(w[:n])))
+        assert np.array_equal(part.view(np.uint32), whole[:n].view(np.uint32)), n
+    _, _, ref = oracle_token(orc, sl, host(X[7].float()), ids=ids[7], w=w[7])
+    assert rel_l2(whole[7], ref) <= LAYER_TOL
+    assert sl.layer.prefill_status() == 0
+
+
 def test_prefill_rejects_unsupported_widths(wm):
     """Prefill needs H, I and the shared width to be multiples of 256."""
     from winmoe_amd import synth

@@ -3,19 +3,19 @@
 // instances, the prefill launcher) and wm_prefill_kq.hip (K-quant instances).
 // Internal; not part of the public ABI.
 //
-// One workgroup of 8 waves per CU works through a static list of items: item
-// j of a launch is (pass, block of matrix rows), and workgroup b takes items
-// k, k + grid, k + 2 grid, ... with k = pf_item_slot(b) (the row blocks of a
-// pass on workgroups of one XCD).
+// One workgroup of 8 waves per CU, or two of 4 (gm_waves), work through a
+// static list of items: item j of a launch is (pass, block of matrix rows),
+// and workgroup b takes items k, k + grid, k + 2 grid, ... with k =
+// pf_item_slot(b) (the row blocks of a pass on workgroups of one XCD).
 //
 // The matrix columns are cut into slices, one per wave (groups of waves when
-// there are fewer than 8 slices: each group then takes its own 16-row tiles).
+// there are fewer slices than waves: each group then takes its own 16-row tiles).
 // A wave keeps the activations of its slice, for all pairs of the pass, in
 // registers as MFMA operands for the whole item, and streams its slice of
 // every row tile: 16 rows x KC columns of raw blocks per ring slot, filled by
 // LDS-DMA of its own, read into registers and refilled at once, so a wave
 // waits for its own loads only and nearly the whole ring is always in flight.
-// Eight waves together read 16 whole rows, a contiguous piece of memory.  The
+// The waves together read 16 whole rows, a contiguous piece of memory.  The
 // waves' partial sums of a tile meet in LDS (one barrier per tile), are added
 // in slice order and leave as the item's outputs.
 //
@@ -84,8 +84,6 @@ constexpr int GM_M = 32;
 constexpr int GM_REC = 64;
 
 constexpr int GM_ROWS = 128;          // matrix rows per gate/up item; columns per activation scale of down
-constexpr int GM_CW = 8;              // waves
-constexpr int GM_THREADS = 64 * GM_CW;
 constexpr int GM_KC = 256;            // columns per super-block (Q8_0: 8 blocks)
 constexpr int GM_SLD = GM_ROWS + 16;  // floats per pair in the SwiGLU staging (rows 16 banks apart)
 
@@ -103,14 +101,15 @@ constexpr int gm_granules(int wt, int nsb) {
     return ((bytes + 2 * mis + 15) / 16) | 1;
 }
 
-// LDS bytes with s ring slots per wave, passes of m pairs, slots of nsb x 256 columns.
-constexpr int gm_lds(int ahl, int wt, int m, int nsb, int s) {
-    return GM_CW * s * 256 * gm_granules(wt, nsb) + 2 * GM_CW * (m / 16) * 1024 + (ahl == 1 ? m * GM_SLD * 4 : 0);
+// LDS bytes of a workgroup of cw waves with s ring slots each, passes of m
+// pairs, slots of nsb x 256 columns; a CU holds 8 / cw workgroups.
+constexpr int gm_lds(int cw, int ahl, int wt, int m, int nsb, int s) {
+    return cw * s * 256 * gm_granules(wt, nsb) + 2 * cw * (m / 16) * 1024 + (ahl == 1 ? m * GM_SLD * 4 : 0);
 }
 // Ring slots per wave: as many as the LDS holds, up to 4.
-constexpr int gm_slots(int ahl, int wt, int m, int nsb) {
+constexpr int gm_slots(int cw, int ahl, int wt, int m, int nsb) {
     int s = 2;
-    while (s < 4 && gm_lds(ahl, wt, m, nsb, s + 1) <= 163840) s++;
+    while (s < 4 && gm_lds(cw, ahl, wt, m, nsb, s + 1) <= 163840 / (8 / cw)) s++;
     return s;
 }
 
@@ -119,13 +118,14 @@ constexpr int gm_slots(int ahl, int wt, int m, int nsb) {
 // registers).  One rule for both pass sizes: the sums are then the same.
 WM_HD constexpr int gm_slice(bool gateup, int ncol) { return gateup ? (ncol < 512 ? ncol : 512) : (ncol > 2048 ? 512 : 256); }
 
-template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB> struct GmGeo {
+template <int AHL, int WT, int M, int NSB, int CW> struct GmGeo {
     static_assert(M == 16 || M == 32, "pass size");
     static_assert(NSB == 1 || NSB == 2, "super-blocks per ring slot");
-    static_assert(NMAT == 1, "a ring slot holds rows of one matrix");
+    static_assert(CW == 4 || CW == 8, "waves");
     static constexpr bool KQ = WT != Q8_0;
     static constexpr bool GU = AHL == 1;                                // gate/up (else down)
-    static_assert(NSUB == (GU ? 2 : 1), "gate and up tiles in turn; down tiles");
+    static constexpr int NSUB = GU ? 2 : 1;                             // gate and up tiles in turn; down tiles
+    static constexpr int THREADS = 64 * CW;
     static constexpr int MT = M / 16;                                   // row tiles of 16 pairs
     static constexpr int KC = GM_KC * NSB;                              // columns per ring slot
     static constexpr int CHUNK = KQ ? NSB * block_bytes(WT) : KC / 32 * 34;   // bytes of a row's slot chunk
@@ -134,13 +134,13 @@ template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB> struct GmGeo {
     static constexpr int RSLOT = 16 * GR;                               // LDS bytes of a row's chunk
     static constexpr int SLOT = 16 * RSLOT;
     static constexpr int NI = (16 * GR + 63) / 64;                      // DMA instructions per slot
-    static constexpr int S = gm_slots(AHL, WT, M, NSB);
-    static constexpr int PART = GM_CW * MT * 1024;                      // partial sums of one tile per wave
-    static constexpr int PBASE = GM_CW * S * SLOT;
+    static constexpr int S = gm_slots(CW, AHL, WT, M, NSB);
+    static constexpr int PART = CW * MT * 1024;                         // partial sums of one tile per wave
+    static constexpr int PBASE = CW * S * SLOT;
     static constexpr int STG = PBASE + 2 * PART;                        // gate/up: M pairs x 128 rows fp32
     static constexpr int LDS = STG + (GU ? M * GM_SLD * 4 : 0);
     static_assert(KQ || GR * 16 == CHUNK, "Q8_0 chunks are whole granules");
-    static_assert(LDS <= 163840 && LDS == gm_lds(AHL, WT, M, NSB, S), "LDS");
+    static_assert(LDS <= 163840 / (8 / CW) && LDS == gm_lds(CW, AHL, WT, M, NSB, S), "LDS");
     static_assert((S - 1) * NI < 64, "vmcnt");
 };
 
@@ -554,18 +554,18 @@ WM_DEV f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f3
 // SwiGLU epilogue.  AHL = 2: down (activations: the pairs' SwiGLU outputs as
 // hi + lo), fp32 output.  WT: the weight format of every matrix the launch
 // reads; M: pairs per pass; NSB: 256-column super-blocks per ring slot.
-template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB>
-__global__ __launch_bounds__(GM_THREADS) void k_pf_gemm(PfGemm a) {
-#if defined(__HIP_DEVICE_COMPILE__)      // the host pass only needs the launch stub (buffer resources are device types)
-    typedef GmGeo<NMAT, AHL, NSUB, WT, M, NSB> G;
+//
+// The items of one launch list (n_r routed ones, then the shared ones, up to
+// n_items) that this workgroup takes: k0, k0 + grid, ...
+#if defined(__HIP_DEVICE_COMPILE__)      // (buffer resources are device types)
+template <int AHL, int WT, int M, int NSB, int CW>
+WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int k0) {
+    typedef GmGeo<AHL, WT, M, NSB, CW> G;
     typedef KqRow<WT> F;
-    constexpr int S = G::S, MT = G::MT, NI = G::NI, MSL = G::MSL;
+    constexpr int S = G::S, MT = G::MT, NI = G::NI, MSL = G::MSL, NSUB = G::NSUB;
     extern __shared__ __attribute__((aligned(16))) uint8_t gsm[];
     // the wave index is uniform: readfirstlane lets the compiler keep what depends on it in SGPRs
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
-    const int n_rp = a.npass[0], n_sp = a.npass[1];
-    const int n_r = a.sel == 2 ? 0 : n_rp * a.nrb_r, n_items = n_r + (a.sel == 1 ? 0 : n_sp * a.nrb_s);
-    const int k0 = pf_item_slot((int)blockIdx.x, (int)gridDim.x, a.sel == 2 ? a.nrb_s : a.nrb_r);
     if (k0 >= n_items) return;
 
     // item i of this workgroup: pass, first matrix row
@@ -583,7 +583,7 @@ __global__ __launch_bounds__(GM_THREADS) void k_pf_gemm(PfGemm a) {
         return true;
     };
     // this wave's slice and row group; a step is 16 rows of each group
-    const int nsl = 1 << a.lsl, sl = wave & (nsl - 1), rgrp = wave >> a.lsl, nrg = GM_CW >> a.lsl;
+    const int nsl = 1 << a.lsl, sl = wave & (nsl - 1), rgrp = wave >> a.lsl, nrg = CW >> a.lsl;
     const int nsteps = a.rows_item / (16 * nrg);
     const int ns = MSL == 2 ? a.ns : 1;
     const uint32_t rb = (uint32_t)a.rb;
@@ -618,9 +618,16 @@ __global__ __launch_bounds__(GM_THREADS) void k_pf_gemm(PfGemm a) {
         lds8_t* dst = ring + islot * G::SLOT;
         const uint32_t colb = (uint32_t)((sl * ns + isl) * G::CHUNK);
         const uint32_t soff = (uint32_t)irow * rb + (colb & ~15u);
+        // The lanes past a slot's last granule stay out of its last
+        // instruction.  The lane number is opaque at each use: a compiler that
+        // knows two of these conditions equal may run the code between them
+        // once for either side, and a DMA whose lanes are so split writes to
+        // one side's address.
+        int ln = lane;
+        asm volatile("" : "+v"(ln));
 #pragma unroll
         for (int t = 0; t < NI; t++)
-            if (16 * G::GR >= 64 * (t + 1) || lane < 16 * G::GR - 64 * t)
+            if (16 * G::GR >= 64 * (t + 1) || ln < 16 * G::GR - 64 * t)
                 __builtin_amdgcn_raw_ptr_buffer_load_lds(NSUB == 2 && imat ? rW1 : rW0, (lds_void*)(dst + 1024 * t), 16,
                                                          voff[t], soff, 0, 0);
         islot = islot + 1 == S ? 0 : islot + 1;
@@ -643,18 +650,22 @@ __global__ __launch_bounds__(GM_THREADS) void k_pf_gemm(PfGemm a) {
 
     // ---- items: the record's parts this lane uses, the activations
     // outputs of a tile: thread tid sums position tid & 255 of row tile
-    // tmt, that is pair om of the pass and row orow of the 16
-    const int tmt = MT == 2 ? tid >> 8 : 0, om = 16 * tmt + 4 * ((tid & 255) >> 6) + (tid & 3), orow = (tid >> 2) & 15;
+    // tmt + q, that is pair om + 16 q of the pass and row orow of the 16
+    constexpr int NO = CW == 4 ? MT : 1;
+    const int tmt = CW == 8 && MT == 2 ? tid >> 8 : 0, om = 16 * tmt + 4 * ((tid & 255) >> 6) + (tid & 3), orow = (tid >> 2) & 15;
     struct Rec {
-        int n, own, xe;                // pairs; this thread's output pair and its x exponent
+        int n, own[NO], xe[NO];        // pairs; this thread's output pairs and their x exponents
         int pid[MT];                   // pair of operand row c
         int4 pq[MT];                   // down: pairs of accumulator rows 4g .. 4g + 3
     };
     auto load_rec = [&](int pass, Rec& r) __attribute__((always_inline)) {
         const int32_t* p = a.recs + (int64_t)pass * GM_REC;
         r.n = ((cint_t*)a.recs)[(int64_t)pass * GM_REC + 1];
-        r.own = p[4 + om];
-        r.xe = G::GU ? (int)((const int8_t*)(p + 4 + GM_M))[om] : 0;
+#pragma unroll
+        for (int q = 0; q < NO; q++) {
+            r.own[q] = p[4 + om + 16 * q];
+            r.xe[q] = G::GU ? (int)((const int8_t*)(p + 4 + GM_M))[om + 16 * q] : 0;
+        }
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
             r.pid[mt] = p[4 + 16 * mt + c];
@@ -840,31 +851,33 @@ __global__ __launch_bounds__(GM_THREADS) void k_pf_gemm(PfGemm a) {
         gm_bar();
         pbuf ^= 1;
         // r: row group of this thread's q-th output
-        auto reduce = [&](int r) __attribute__((always_inline)) {
-            const float* p = pb + (((r << a.lsl) * MT + tmt) * 256) + (tid & 255);
+        auto reduce = [&](int r, int q) __attribute__((always_inline)) {
+            const float* p = pb + (((r << a.lsl) * MT + tmt + q) * 256) + (tid & 255);
             float v;
-            if (a.lsl == 3) v = sum_slices<8, MT * 256>(p);
+            if (CW == 8 && a.lsl == 3) v = sum_slices<8, MT * 256>(p);
             else if (a.lsl == 2) v = sum_slices<4, MT * 256>(p);
             else if (a.lsl == 1) v = sum_slices<2, MT * 256>(p);
             else v = p[0];
             const int row = 16 * (st * nrg + r) + orow;
             if constexpr (G::GU) {
-                float* sp = stg + om * GM_SLD + row;
+                float* sp = stg + (om + 16 * q) * GM_SLD + row;
                 if (mat == 0) *sp = v;
                 else {
-                    const float xs = ldexpf(1.0f, cur.xe);
+                    const float xs = ldexpf(1.0f, cur.xe[q]);
                     *sp = silu_mul(*sp * xs, v * xs);
                 }
             } else {
-                if (om < cur.n) a.y[(int64_t)cur.own * a.y_ld + crow + row] = v;
+                if (om + 16 * q < cur.n) a.y[(int64_t)cur.own[q] * a.y_ld + crow + row] = v;
             }
         };
-        if constexpr (MT == 2) {
-            for (int r = 0; r < nrg; r++) reduce(r);
+        if constexpr (CW == 4 || MT == 2) {
+            for (int r = 0; r < nrg; r++)
+#pragma unroll
+                for (int q = 0; q < NO; q++) reduce(r, q);
         } else if (nrg == 1) {
-            if ((tid >> 8) == (st & 1)) reduce(0);           // 4 waves each, in turn
+            if ((tid >> 8) == (st & 1)) reduce(0, 0);        // 4 waves each, in turn
         } else {
-            for (int r = tid >> 8; r < nrg; r += 2) reduce(r);
+            for (int r = tid >> 8; r < nrg; r += 2) reduce(r, 0);
         }
     };
 
@@ -885,7 +898,8 @@ __global__ __launch_bounds__(GM_THREADS) void k_pf_gemm(PfGemm a) {
             asm volatile("" : "+v"(nxt.pid[mt]));
             if constexpr (!G::GU) asm volatile("" : "+v"(nxt.pq[mt].x), "+v"(nxt.pq[mt].y), "+v"(nxt.pq[mt].z), "+v"(nxt.pq[mt].w));
         }
-        asm volatile("" : "+v"(nxt.own), "+v"(nxt.xe));
+#pragma unroll
+        for (int q = 0; q < NO; q++) asm volatile("" : "+v"(nxt.own[q]), "+v"(nxt.xe[q]));
         f32x4 acc[MT];
         for (int st = 0;; st++) {
 #pragma unroll
@@ -905,10 +919,10 @@ __global__ __launch_bounds__(GM_THREADS) void k_pf_gemm(PfGemm a) {
         if (nok) load_act(nxt);
         finish(NSUB - 1, nsteps - 1, acc);
         if constexpr (G::GU) {
-            // wave w: pairs w, w + 8, ..: scale by a power of two, split into hi + lo
+            // wave w: pairs w, w + CW, ..: scale by a power of two, split into hi + lo
             gm_bar();
             const int32_t* rec = a.recs + (int64_t)cp * GM_REC;
-            for (int m = wave; m < cur.n; m += GM_CW) {
+            for (int m = wave; m < cur.n; m += CW) {
                 const float2 v = *(const float2*)(stg + m * GM_SLD + 2 * lane);
                 float mx = fmaxf(fabsf(v.x), fabsf(v.y));
                 mx = fmaxf(mx, dpp_f32<DPP_ROR8>(mx));
@@ -939,24 +953,52 @@ __global__ __launch_bounds__(GM_THREADS) void k_pf_gemm(PfGemm a) {
         nok = item(ci + 1, np, nrow);
         if (nok) load_rec(np, nxt);
     }
+}
+#endif
+
+// A CU holds 8 waves either way: one workgroup of 8, or two of 4.
+template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB, int CW = 8>
+__global__ __launch_bounds__(64 * CW, 2) void k_pf_gemm(PfGemm a) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int n_rp = a.npass[0], n_r = a.sel == 2 ? 0 : n_rp * a.nrb_r;
+    pf_gemm_items<AHL, WT, M, NSB, CW>(a, n_rp, n_r, n_r + (a.sel == 1 ? 0 : a.npass[1] * a.nrb_s),
+                                       pf_item_slot((int)blockIdx.x, (int)gridDim.x, a.sel == 2 ? a.nrb_s : a.nrb_r));
 #endif
 }
 
-template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB = 1>
-int launch_pf_gemm(const PfGemm& g, int n_wg, hipStream_t s) {
-    typedef GmGeo<NMAT, AHL, NSUB, WT, M, NSB> G;
-    PfGemm h = g;
-    const int slice = gm_slice(G::GU, g.ncol), nsl = g.ncol / slice;
+// Slices and ring slots of a launch; false if the shape does not fit.
+template <class G> bool pf_gemm_plan(PfGemm& h, int cw) {
+    const int slice = gm_slice(G::GU, h.ncol), nsl = h.ncol / slice;
     h.ns = slice / G::KC;
     h.lsl = nsl == 1 ? 0 : nsl == 2 ? 1 : nsl == 4 ? 2 : 3;
-    // whole slots and slices; a step's rows divide an item's
-    if (slice % G::KC || h.ns > G::MSL || g.ncol % slice || (1 << h.lsl) != nsl || g.rows_item % 128)
-        return (int)hipErrorInvalidValue;
-    hipError_t e = hipFuncSetAttribute((const void*)k_pf_gemm<NMAT, AHL, NSUB, WT, M, NSB>,
+    // whole slots and slices, no more slices than waves; a step's rows divide an item's
+    return !(slice % G::KC || h.ns > G::MSL || h.ncol % slice || (1 << h.lsl) != nsl || nsl > cw || h.rows_item % 128);
+}
+
+// Waves of a workgroup: 4, two workgroups to a CU, when the row has no more
+// than 4 slices; one of 8 else.  The waves of a workgroup meet once per tile,
+// and those of the two workgroups do not wait for each other: one computes
+// while the other is at its barrier or waits for its partial sums.  us per
+// batch with one workgroup of 8 / two of 4 (the same bits): H 4096, I 1024
+// (down alone), Q8_0 top-10 at 512 tokens 1326 / 1312, at 4096 tokens 4018 /
+// 3719; Q4_K, Q6_K top-3 at 512 tokens 995 / 950, at 2000 1656 / 1582; H 2048,
+// I 512 (both), Q8_0 top-4 of 64 at 1001 tokens 197 / 179.
+WM_HD inline int gm_waves(bool gateup, int ncol) { return ncol / gm_slice(gateup, ncol) <= 4 ? 4 : 8; }
+
+template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB, int CW>
+int launch_pf_gemm_cw(PfGemm h, int n_wg, hipStream_t s) {
+    typedef GmGeo<AHL, WT, M, NSB, CW> G;
+    if (!pf_gemm_plan<G>(h, CW)) return (int)hipErrorInvalidValue;
+    hipError_t e = hipFuncSetAttribute((const void*)k_pf_gemm<NMAT, AHL, NSUB, WT, M, NSB, CW>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((k_pf_gemm<NMAT, AHL, NSUB, WT, M, NSB>), dim3(n_wg), dim3(GM_THREADS), G::LDS, s, h);
+    hipLaunchKernelGGL((k_pf_gemm<NMAT, AHL, NSUB, WT, M, NSB, CW>), dim3(n_wg * (8 / CW)), dim3(64 * CW), G::LDS, s, h);
     return (int)hipGetLastError();
+}
+template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB = 1>
+int launch_pf_gemm(const PfGemm& g, int n_wg, hipStream_t s) {
+    if (gm_waves(AHL == 1, g.ncol) == 4) return launch_pf_gemm_cw<NMAT, AHL, NSUB, WT, M, NSB, 4>(g, n_wg, s);
+    return launch_pf_gemm_cw<NMAT, AHL, NSUB, WT, M, NSB, 8>(g, n_wg, s);
 }
 
 // The K-quant instances (wm_prefill_kq.hip): gate/up and down of Q2_K ..

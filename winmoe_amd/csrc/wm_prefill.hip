@@ -25,6 +25,7 @@
 #include <hip/hip_runtime.h>
 #include <stdint.h>
 
+#include <algorithm>
 #include <type_traits>
 
 #include "../../include/winmoe_hip.h"
@@ -626,6 +627,20 @@ int launch_prefill_gateup(const PrefillArgs& a, hipStream_t s) {
     return launch_split(a.pass_m, true, {a.gt, a.H}, {a.sgt, a.H}, a.has_shared, g, a.n_wg, s);
 }
 
+// Rows of a down item: 512 read a pass's activations least often; a batch
+// whose items are then fewer than two rounds of the workgroups (two per CU)
+// takes 256, and 128 below half a round, so that the rounds come out even.
+// us per batch, 512 / 256 / 128 rows: 8 tokens, 64 experts, H 2048 (0.3
+// rounds) 75 / 61 / 57; 1001 tokens, 64 experts, H 2048 (1.5) 179 / 177 /
+// 195; 300 tokens, 128 experts, H 2048 (1.6) 165 / 158 / 166; 90 tokens, 256
+// experts, H 4096 (3.5) 222 / 231 / 238; 4096 tokens Q8_0 3719 / 3841 / 4245.
+static int down_rows(const PrefillArgs& a) {
+    const int64_t pairs = (int64_t)a.T * a.K, m = a.pass_m;
+    const int64_t passes = std::min<int64_t>(pairs, a.E) + pairs / m + (a.has_shared ? a.T / m : 0);
+    const int64_t items = passes * a.H / 512, grid = 2 * (int64_t)a.n_wg;
+    return a.H % 512 || items < 2 * grid ? (2 * items < grid ? 128 : 256) : 512;
+}
+
 int launch_prefill_down(const PrefillArgs& a, hipStream_t s) {
     PfGemm g = {};
     g.w0 = a.down; g.w1 = a.down; g.st0 = g.st1 = a.dstride;
@@ -634,7 +649,7 @@ int launch_prefill_down(const PrefillArgs& a, hipStream_t s) {
     g.mb_s = a.has_shared ? (int32_t)matrix_bytes(a.sdt, a.H, a.Is) : g.mb_r;
     g.a_hi = a.act_hi; g.a_lo = a.act_lo; g.a_ld = a.act_stride; g.a_sc = a.act_sc; g.sc_ld = a.act_stride / 128;
     g.T = a.T; g.K = a.K;
-    g.rows_item = a.H % 512 == 0 ? 512 : 256;
+    g.rows_item = down_rows(a);
     g.nrb_r = g.nrb_s = a.H / g.rows_item;
     g.recs = a.passes; g.npass = a.pass_count;
     g.y = a.y; g.y_ld = a.H;
