@@ -966,6 +966,25 @@ __global__ __launch_bounds__(64 * CW, 2) void k_pf_gemm(PfGemm a) {
 #endif
 }
 
+// Routed passes in format WT, then the shared expert's in format SWT, in one
+// launch: the shared items go on where the routed ones ended, so that the
+// workgroups without an item of the last round take them.  A launch of their
+// own left most of the chip idle at both ends: 2 passes of gate/up are 16
+// items, 38 us.  23 tokens through 512 experts of H 4096, I 1024, Q4_K, Q6_K,
+// top-3, Q8_0 shared: 238 us per batch with two launches, 195 with one (the
+// same bits).
+template <int AHL, int WT, int M, int NSB, int SWT, int CW>
+__global__ __launch_bounds__(64 * CW, 2) void k_pf_gemm2(PfGemm r, PfGemm s) {
+#if defined(__HIP_DEVICE_COMPILE__)
+    const int n_rp = r.npass[0], n_r = n_rp * r.nrb_r, grid = (int)gridDim.x;
+    const int k0 = pf_item_slot((int)blockIdx.x, grid, r.nrb_r);
+    pf_gemm_items<AHL, WT, M, NSB, CW>(r, n_rp, n_r, n_r, k0);
+    __syncthreads();                             // the ring and the staging change hands
+    const int first = k0 - n_r % grid;
+    pf_gemm_items<AHL, SWT, M, 1, CW>(s, n_rp, 0, s.npass[1] * s.nrb_s, first < 0 ? first + grid : first);
+#endif
+}
+
 // Slices and ring slots of a launch; false if the shape does not fit.
 template <class G> bool pf_gemm_plan(PfGemm& h, int cw) {
     const int slice = gm_slice(G::GU, h.ncol), nsl = h.ncol / slice;
@@ -1001,9 +1020,31 @@ int launch_pf_gemm(const PfGemm& g, int n_wg, hipStream_t s) {
     return launch_pf_gemm_cw<NMAT, AHL, NSUB, WT, M, NSB, 8>(g, n_wg, s);
 }
 
+template <int AHL, int WT, int M, int NSB, int SWT, int CW>
+int launch_pf_gemm2_cw(PfGemm h, PfGemm hs, int n_wg, hipStream_t s) {
+    typedef GmGeo<AHL, WT, M, NSB, CW> GR;
+    typedef GmGeo<AHL, SWT, M, 1, CW> GS;
+    if (!pf_gemm_plan<GR>(h, CW) || !pf_gemm_plan<GS>(hs, CW)) return (int)hipErrorInvalidValue;
+    constexpr int lds = GR::LDS > GS::LDS ? GR::LDS : GS::LDS;
+    hipError_t e = hipFuncSetAttribute((const void*)k_pf_gemm2<AHL, WT, M, NSB, SWT, CW>,
+                                       hipFuncAttributeMaxDynamicSharedMemorySize, lds);
+    if (e != hipSuccess) return (int)e;
+    hipLaunchKernelGGL((k_pf_gemm2<AHL, WT, M, NSB, SWT, CW>), dim3(n_wg * (8 / CW)), dim3(64 * CW), lds, s, h, hs);
+    return (int)hipGetLastError();
+}
+template <int AHL, int WT, int M, int NSB, int SWT>
+int launch_pf_gemm2(const PfGemm& r, const PfGemm& sh, int n_wg, hipStream_t s) {
+    if (gm_waves(AHL == 1, r.ncol) == 4 && gm_waves(AHL == 1, sh.ncol) == 4)
+        return launch_pf_gemm2_cw<AHL, WT, M, NSB, SWT, 4>(r, sh, n_wg, s);
+    return launch_pf_gemm2_cw<AHL, WT, M, NSB, SWT, 8>(r, sh, n_wg, s);
+}
+
 // The K-quant instances (wm_prefill_kq.hip): gate/up and down of Q2_K ..
 // Q6_K, for passes of m = 16 or 32 pairs.  Returns hipErrorInvalidValue for
 // another combination.
 int launch_pf_gemm_kq(int m, bool gateup, int wt, const PfGemm& g, int n_wg, hipStream_t s);
+// Routed K-quant passes and the shared expert's Q8_0 ones in one launch
+// (gate/up, or passes of 16: down of 32 has no registers left for both).
+int launch_pf_gemm_kq_q8(int m, bool gateup, int wt, const PfGemm& g, const PfGemm& sh, int n_wg, hipStream_t s);
 
 }  // namespace wm
