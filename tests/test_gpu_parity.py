@@ -577,6 +577,41 @@ def test_prefill_batch_split(wm, orc, H, I, types, sh_inter):
     assert sl.layer.prefill_status() == 0
 
 
+@pytest.mark.parametrize("T,K,E", [(70, 1, 5), (1024, 8, 64), (1025, 8, 300), (4096, 10, 1000), (4097, 11, 17),
+                                   (9000, 8, 1024)])
+def test_prefill_grouping_limits(wm, T, K, E):
+    """The grouping at the sizes where it leaves registers (8192 pairs), LDS
+    (45056 pairs, 8192 tokens, 4096 routed passes), with ids outside [0, E):
+    hit counters, the status word, and every 97th token against a batch of
+    those tokens alone, bit for bit."""
+    import torch
+    from winmoe_amd import _lib, synth
+    cfg = synth.LayerConfig(f"pf_group_{T}_{K}_{E}", E=E, K=K, H=256, I=256, types=(Q8_0, Q8_0, Q8_0),
+                            shared_types=(Q8_0,) * 3, shared_inter=256, shared_gate_inp=True, tokens=1,
+                            routing="zipf", x_dtype="bf16", seed=9)
+    sl = synth.build_layer(cfg, max_tokens=T)
+    sl.layer.desc.flags |= _lib.FLAG_PREFILL_PASS16
+    X = synth.make_hidden(cfg, tokens=T)
+    rng = np.random.default_rng(T + K)
+    ids = rng.integers(0, E, (T, K)).astype(np.int32)
+    ids[::50, 0] = rng.choice([-1, E, E + 1000], len(ids[::50, 0]))
+    w = rng.random((T, K)).astype(np.float32)
+    case(f"prefill grouping T={T} K={K} E={E}")
+    whole = host(sl.layer.prefill_forced(X, dev(ids), dev(w)))
+    from winmoe_amd.moe import load
+    import ctypes as C
+    off = [C.c_int64() for _ in range(3)]
+    load().wm_prefill_workspace_routing(C.byref(sl.layer.desc), sl.layer.pf_tokens, *[C.byref(o) for o in off])
+    o = off[2].value
+    hits = host(sl.layer.pf_ws[o:o + 4 * E].view(torch.int32))
+    ok = ids[(ids >= 0) & (ids < E)]
+    assert np.array_equal(hits, np.bincount(ok, minlength=E))
+    assert sl.layer.prefill_status() & 2
+    pick = np.arange(0, T, 97)
+    part = host(sl.layer.prefill_forced(X[::97].contiguous(), dev(ids[pick]), dev(w[pick])))
+    assert np.array_equal(part.view(np.uint32), whole[pick].view(np.uint32))
+
+
 def test_prefill_rejects_unsupported_widths(wm):
     """Prefill needs H, I and the shared width to be multiples of 256."""
     from winmoe_amd import synth

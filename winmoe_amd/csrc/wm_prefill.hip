@@ -9,10 +9,11 @@
 //   k_pf_router    the same for other widths and alignments (tiles of 16
 //                  tokens x 16 experts, each lane one of the 16 FMA chains of
 //                  4 x 4 (token, expert) pairs)
-//   k_pf_topk      one wave per token: K-pass arg-max + softmax
+//   k_pf_tokens    per token: K-pass arg-max + softmax (or the caller's
+//                  routing), x as fp16 times a power of two, the shared
+//                  expert's gate
 //   k_pf_group     counting sort of the pairs by expert; passes of <= 16
 //                  or 32 pairs of one expert (prefill_pass_size)
-//   k_pf_xpack     x as fp16 times a power of two per token
 //   k_pf_gemm      gate and up + SwiGLU on fp16 MFMA, persistent: one
 //                  workgroup per CU streams (pass, 128-row block) items
 //                  through an LDS-DMA ring; the SwiGLU output is stored as
@@ -265,27 +266,6 @@ __global__ __launch_bounds__(256) void k_pf_router_m(const uint16_t* __restrict_
 
 // ------------------------------------------------------------------ top-K, forced routing, grouping
 
-__global__ __launch_bounds__(256) void k_pf_topk(const float* __restrict__ logits, int T, int E, int K,
-                                                 int32_t* __restrict__ ids, float* __restrict__ w,
-                                                 uint32_t* __restrict__ hits, int32_t* __restrict__ status) {
-    const int t = blockIdx.x * WAVES + (threadIdx.x >> 6);
-    if (t >= T) return;                       // whole waves
-    wave_topk<false>(logits + (int64_t)t * E, E, K, ids + (int64_t)t * K, w + (int64_t)t * K, hits, status,
-                     threadIdx.x & 63);
-}
-
-__global__ __launch_bounds__(256) void k_pf_forced(const int32_t* __restrict__ fids, const float* __restrict__ fw,
-                                                   int n, int E, int32_t* __restrict__ ids, float* __restrict__ w,
-                                                   uint32_t* __restrict__ hits, int32_t* __restrict__ status) {
-    const int p = blockIdx.x * 256 + threadIdx.x;
-    if (p >= n) return;
-    const int e = fids[p];
-    ids[p] = e;
-    w[p] = fw[p];
-    if (e >= 0 && e < E) atomicAdd(hits + e, 1u);
-    else atomicOr(status, WM_STATUS_BAD_EXPERT_ID);
-}
-
 // Exclusive prefix sums of (a, b) over the 1024 threads of a workgroup; the
 // totals go to *tot.  wsum: 16 x 2 ints of LDS.
 WM_DEV int2 block_excl_scan2(int2 v, int* wsum, int2* tot) {
@@ -320,46 +300,58 @@ WM_DEV int2 block_excl_scan2(int2 v, int* wsum, int2* tot) {
 }
 
 // Sizes for which k_pf_group keeps its data on chip: the pairs' expert ids
-// in registers (up to PG_REG per thread), the sorted pair list and the
-// tokens' exponents in LDS; larger batches read them from global memory.
-constexpr int PG_REG = 8, PG_SORT = 10240, PG_XEXP = 2048;
+// in registers (up to PG_REG per thread), the sorted pair list (16-bit
+// entries) and the tokens' exponents (a byte each) in LDS, and the experts of
+// the passes; larger batches read them from global memory, or search.
+constexpr int PG_REG = 8, PG_SORT = 45056, PG_XEXP = 8192, PG_MAP = 4096;
 
 // One workgroup: pairs grouped by expert (order inside an expert is free:
 // every pair's output row is computed independently of the others), then
 // cut into pass records of at most pm pairs (16 or 32): routed passes first,
 // in expert order, then the shared expert's; pass_count = {routed passes,
 // shared passes}.  A record also carries the x scale of each pair's token.
-__global__ __launch_bounds__(1024) void k_pf_group(const int32_t* __restrict__ ids, int T, int K, int E, int has_shared,
-                                                   int pm,
-                                                   int32_t* __restrict__ offsets, int32_t* __restrict__ sorted,
-                                                   int32_t* __restrict__ passes, int32_t* __restrict__ pass_count,
-                                                   const int32_t* __restrict__ xexp) {
+// The experts' hit counters are raised here, by one add per expert: 4004
+// pairs over 64 experts spent 10 us on device atomics to 64 words.
+//
+// Bound by latency: one workgroup, so the records are written by 8 threads
+// each (16-byte pieces of a pass side by side), a pair's token is a multiply
+// by kmul = ceil(2^32 / K) instead of a division, and ids are read PG_REG to
+// a thread at a time.
+__global__ __launch_bounds__(1024) void k_pf_group(const int32_t* __restrict__ ids, int T, int K, uint32_t kmul, int E,
+                                                   int has_shared, int pm, int32_t* __restrict__ offsets,
+                                                   int32_t* __restrict__ sorted, int32_t* __restrict__ passes,
+                                                   int32_t* __restrict__ pass_count, const int32_t* __restrict__ xexp,
+                                                   uint32_t* __restrict__ hits) {
     __shared__ int cnt[1025];
     __shared__ int off[1026];
     __shared__ int pbase[1026];
     __shared__ int wsum[32];
-    __shared__ int srt[PG_SORT];
-    __shared__ int xe[PG_XEXP];
+    __shared__ uint16_t srt[PG_SORT];
+    __shared__ uint16_t pexp[PG_MAP];
+    __shared__ uint8_t xe[PG_XEXP];
     const int tid = threadIdx.x, P = T * K, G = E + 1;      // group E: the shared expert (empty without one)
     const bool reg = P <= 1024 * PG_REG, lsort = P + (has_shared ? T : 0) <= PG_SORT, lxe = T <= PG_XEXP;
-    // the ids and exponents are read once, together
+    // the ids and exponents are read once, together (more than PG_REG ids to a thread: again for the scatter)
     int ev[PG_REG];
+    auto load_ids = [&](int base) __attribute__((always_inline)) {
 #pragma unroll
-    for (int i = 0; i < PG_REG; i++) ev[i] = reg && tid + 1024 * i < P ? ids[tid + 1024 * i] : -1;
+        for (int i = 0; i < PG_REG; i++) {
+            const int p = base + tid + 1024 * i;
+            ev[i] = p < P ? ids[p] : -1;
+            if (ev[i] >= E) ev[i] = -1;
+        }
+    };
+    load_ids(0);
     if (lxe)
-        for (int t = tid; t < T; t += 1024) xe[t] = xexp[t];
+        for (int t = tid; t < T; t += 1024) xe[t] = (uint8_t)xexp[t];
     for (int e = tid; e < E; e += 1024) cnt[e] = 0;
     if (tid == 0) cnt[E] = has_shared ? T : 0;
     __syncthreads();
-    if (reg) {
+    for (int base = 0; base < P; base += 1024 * PG_REG) {
+        if (base) load_ids(base);
 #pragma unroll
         for (int i = 0; i < PG_REG; i++)
-            if (ev[i] >= 0 && ev[i] < E) atomicAdd(&cnt[ev[i]], 1);
-    } else {
-        for (int p = tid; p < P; p += 1024) {
-            const int e = ids[p];
-            if (e >= 0 && e < E) atomicAdd(&cnt[e], 1);
-        }
+            if (ev[i] >= 0) atomicAdd(&cnt[ev[i]], 1);
     }
     __syncthreads();
     // pair offsets and pass bases of the groups, 1024 groups per round
@@ -367,6 +359,7 @@ __global__ __launch_bounds__(1024) void k_pf_group(const int32_t* __restrict__ i
     for (int base = 0; base < G; base += 1024) {
         const int e = base + tid;
         const int n = e < G ? cnt[e] : 0;
+        if (e < E && n) hits[e] += (uint32_t)n;
         int2 tot;
         const int2 ex = block_excl_scan2(make_int2(n, (n + pm - 1) / pm), wsum, &tot);
         if (e < G) {
@@ -387,77 +380,94 @@ __global__ __launch_bounds__(1024) void k_pf_group(const int32_t* __restrict__ i
         pass_count[0] = pbase[E];
         pass_count[1] = pbase[G] - pbase[E];
     }
+    const int npass = pbase[G], nrouted = pbase[E];
+    const bool map = nrouted <= PG_MAP;
+    if (map)
+        for (int e = tid; e < E; e += 1024)
+            for (int q = pbase[e]; q < pbase[e + 1]; q++) pexp[q] = (uint16_t)e;
     // the sorted list: in LDS when it fits, else in global memory
-    if (reg) {
+    auto put = [&](int pos, int p) __attribute__((always_inline)) {
+        if (lsort) srt[pos] = (uint16_t)p;
+        else sorted[pos] = p;
+    };
+    for (int base = 0; base < P; base += 1024 * PG_REG) {
+        if (!reg) load_ids(base);
 #pragma unroll
-        for (int i = 0; i < PG_REG; i++) {
-            const int e = ev[i], p = tid + 1024 * i;
-            if (e >= 0 && e < E) {
-                const int pos = atomicAdd(&cnt[e], 1);
-                if (lsort) srt[pos] = p;
-                else sorted[pos] = p;
-            }
-        }
-    } else {
-        for (int p = tid; p < P; p += 1024) {
-            const int e = ids[p];
-            if (e >= 0 && e < E) {
-                const int pos = atomicAdd(&cnt[e], 1);
-                if (lsort) srt[pos] = p;
-                else sorted[pos] = p;
-            }
-        }
+        for (int i = 0; i < PG_REG; i++)
+            if (ev[i] >= 0) put(atomicAdd(&cnt[ev[i]], 1), base + tid + 1024 * i);
     }
     if (has_shared)
-        for (int t = tid; t < T; t += 1024) {
-            if (lsort) srt[off[E] + t] = P + t;
-            else sorted[off[E] + t] = P + t;
-        }
+        for (int t = tid; t < T; t += 1024) put(off[E] + t, P + t);
     __syncthreads();
-    // one thread per pass: its group by binary search over the pass bases
-    const int npass = pbase[G];
-    for (int q = tid; q < npass; q += 1024) {
-        int lo = 0, hi = G - 1;                  // largest e with pbase[e] <= q
-        while (lo < hi) {
-            const int mid = (lo + hi + 1) >> 1;
-            if (pbase[mid] <= q) lo = mid;
-            else hi = mid - 1;
+    // thread: 4 pairs of a pass
+    for (int it = tid; it < 8 * npass; it += 1024) {
+        const int q = it >> 3, m4 = it & 7;
+        int e = E;
+        if (q < nrouted) {
+            if (map) e = pexp[q];
+            else {
+                int lo = 0, hi = E - 1;          // largest e with pbase[e] <= q
+                while (lo < hi) {
+                    const int mid = (lo + hi + 1) >> 1;
+                    if (pbase[mid] <= q) lo = mid;
+                    else hi = mid - 1;
+                }
+                e = lo;
+            }
         }
-        const int e = lo, first = off[e] + (q - pbase[e]) * pm;
+        const int first = off[e] + (q - pbase[e]) * pm;
         const int mn = min(pm, off[e + 1] - first);
         int32_t* rec = passes + (int64_t)q * GM_REC;
-        rec[0] = e;
-        rec[1] = mn;
-        rec[2] = 0;
-        rec[3] = 0;
-        int prs[GM_M];
+        int prs[4];
+        uint32_t ex = 0;
 #pragma unroll
-        for (int m = 0; m < GM_M; m++) {
-            const int at = first + min(m, mn - 1);
-            prs[m] = lsort ? srt[at] : sorted[at];
+        for (int j = 0; j < 4; j++) {
+            const int at = first + min(4 * m4 + j, mn - 1);
+            prs[j] = lsort ? (int)srt[at] : sorted[at];
         }
 #pragma unroll
-        for (int m4 = 0; m4 < GM_M / 4; m4++) {
-            uint32_t ex = 0;
-#pragma unroll
-            for (int j = 0; j < 4; j++) {
-                const int pr = prs[4 * m4 + j], tok = pair_token(pr, T, K);
-                rec[4 + 4 * m4 + j] = pr;
-                ex |= (uint32_t)((lxe ? xe[tok] : xexp[tok]) & 0xFF) << (8 * j);
-            }
-            rec[4 + GM_M + m4] = (int32_t)ex;
+        for (int j = 0; j < 4; j++) {
+            const int pr = prs[j];
+            const int tok = pr >= P ? pr - P : K == 1 ? pr : (int)__umulhi((uint32_t)pr, kmul);
+            ex |= (uint32_t)((lxe ? (int)xe[tok] : xexp[tok]) & 0xFF) << (8 * j);
         }
+        if (m4 == 0) *(int4*)rec = make_int4(e, mn, 0, 0);
+        *(int4*)(rec + 4 + 4 * m4) = make_int4(prs[0], prs[1], prs[2], prs[3]);
+        rec[4 + GM_M + m4] = (int32_t)ex;
     }
 }
 
-// x bf16 [T][H] -> x16 = fp16(x * 2^-e) with e per token (pf_exp of the
-// token's largest |x|), xexp[t] = e.  bf16 values are exact in fp16 at that
-// scale (8 significant bits, normal range down to 2^-29 of the maximum).
-__global__ __launch_bounds__(256) void k_pf_xpack(const uint16_t* __restrict__ x, int H, uint16_t* __restrict__ x16,
-                                                  int32_t* __restrict__ xexp) {
+// What a batch needs of each token ahead of the expert GEMMs, one workgroup
+// per token, one launch (each was a launch of its own, 5 us apiece):
+//   * its experts and weights: arg-max and softmax of its logits (wave 0), or
+//     the caller's (logits NULL);
+//   * x bf16 [H] -> x16 = fp16(x * 2^-e) with e per token (pf_exp of the
+//     token's largest |x|), xexp[t] = e.  bf16 values are exact in fp16 at
+//     that scale (8 significant bits, normal range down to 2^-29 of the
+//     maximum);
+//   * the shared expert's gate (g not NULL): sigmoid_stable((float) sum_h
+//     g[h] x[h]) with the dot in fp64 (winmoe_inference.c:2005-2009),
+//     fixed-order tree.
+__global__ __launch_bounds__(256) void k_pf_tokens(const uint16_t* __restrict__ x, int H, uint16_t* __restrict__ x16,
+                                                   int32_t* __restrict__ xexp, const float* __restrict__ g,
+                                                   float* __restrict__ sg, const float* __restrict__ logits,
+                                                   const int32_t* __restrict__ fids, const float* __restrict__ fw, int E,
+                                                   int K, int32_t* __restrict__ ids, float* __restrict__ w,
+                                                   int32_t* __restrict__ status) {
     __shared__ float wmax[WAVES];
+    __shared__ double part[256];
     const int t = blockIdx.x, lane = threadIdx.x & 63, wave = threadIdx.x >> 6;
     const uint16_t* xr = x + (int64_t)t * H;
+    if (logits) {
+        if (wave == 0)
+            wave_topk<false>(logits + (int64_t)t * E, E, K, ids + (int64_t)t * K, w + (int64_t)t * K, nullptr, status, lane);
+    } else if ((int)threadIdx.x < K) {
+        const int64_t p = (int64_t)t * K + threadIdx.x;
+        const int e = fids[p];
+        ids[p] = e;
+        w[p] = fw[p];
+        if (e < 0 || e >= E) atomicOr(status, WM_STATUS_BAD_EXPERT_ID);
+    }
     float m = 0.0f;
     for (int c0 = threadIdx.x * 8; c0 < H; c0 += 256 * 8) {
         const u32x4 v = *(const u32x4*)(xr + c0);
@@ -475,6 +485,22 @@ __global__ __launch_bounds__(256) void k_pf_xpack(const uint16_t* __restrict__ x
     r = fmaxf(r, __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), 32)));
     r = fmaxf(r, __builtin_bit_cast(float, __builtin_amdgcn_readlane(__builtin_bit_cast(int, m), 48)));
     if (lane == 0) wmax[wave] = r;
+    if (g) {
+        double acc = 0.0;
+        for (int base = 0; base < H; base += 256 * 16) {
+            float gv[16], xv[16];
+#pragma unroll
+            for (int i = 0; i < 16; i++) {
+                const int h = min(base + (int)threadIdx.x + 256 * i, H - 1);
+                gv[i] = g[h];
+                xv[i] = bf16f(xr[h]);
+            }
+#pragma unroll
+            for (int i = 0; i < 16; i++)
+                if (base + (int)threadIdx.x + 256 * i < H) acc += (double)gv[i] * (double)xv[i];
+        }
+        part[threadIdx.x] = acc;
+    }
     __syncthreads();
     const float M = fmaxf(fmaxf(wmax[0], wmax[1]), fmaxf(wmax[2], wmax[3]));
     const int e = pf_exp(M);
@@ -492,38 +518,18 @@ __global__ __launch_bounds__(256) void k_pf_xpack(const uint16_t* __restrict__ x
         *(u32x4*)(x16 + (int64_t)t * H + c0) = o;
     }
     if (threadIdx.x == 0) xexp[t] = e;
-}
-
-// Shared-expert gate of every token: sigmoid_stable((float) sum_h g[h] x[h])
-// with the dot in fp64 (winmoe_inference.c:2005-2009), fixed-order tree.
-__global__ __launch_bounds__(256) void k_pf_shgate(const uint16_t* __restrict__ x, const float* __restrict__ g, int H,
-                                                   float* __restrict__ sg) {
-    __shared__ double part[256];
-    const int t = blockIdx.x;
-    const uint16_t* xr = x + (int64_t)t * H;
-    double acc = 0.0;
-    for (int base = 0; base < H; base += 256 * 16) {
-        float gv[16], xv[16];
-#pragma unroll
-        for (int i = 0; i < 16; i++) {
-            const int h = min(base + (int)threadIdx.x + 256 * i, H - 1);
-            gv[i] = g[h];
-            xv[i] = bf16f(xr[h]);
-        }
-#pragma unroll
-        for (int i = 0; i < 16; i++)
-            if (base + (int)threadIdx.x + 256 * i < H) acc += (double)gv[i] * (double)xv[i];
-    }
-    part[threadIdx.x] = acc;
-    __syncthreads();
-    for (int m = 128; m >= 1; m >>= 1) {
-        if ((int)threadIdx.x < m) part[threadIdx.x] += part[threadIdx.x + m];
+    if (!g) return;
+    for (int d = 128; d >= 64; d >>= 1) {
+        if ((int)threadIdx.x < d) part[threadIdx.x] += part[threadIdx.x + d];
         __syncthreads();
     }
-    if (threadIdx.x == 0) sg[t] = sigmoid_stable((float)part[0]);
+    if (wave == 0) {
+        double v = part[lane];
+#pragma unroll
+        for (int d = 32; d >= 1; d >>= 1) v += __shfl_down(v, d);
+        if (lane == 0) sg[t] = sigmoid_stable((float)v);
+    }
 }
-
-
 
 // out[t][h] = sum_k w[t][k] y[t*K + k][h] (k order, invalid ids skipped) + gate(t) * y_shared[t][h];
 // 4 consecutive h per thread.
@@ -557,11 +563,7 @@ __global__ __launch_bounds__(256) void k_pf_combine(PrefillArgs a) {
 // ------------------------------------------------------------------ launcher
 
 int launch_prefill_route(const PrefillArgs& a, const int32_t* forced_ids, const float* forced_w, hipStream_t s) {
-    const int P = a.T * a.K;
-    if (forced_ids) {
-        hipLaunchKernelGGL(k_pf_forced, dim3((P + 255) / 256), dim3(256), 0, s, forced_ids, forced_w, P, a.E, a.ids, a.w,
-                           a.hits, a.status);
-    } else {
+    if (!forced_ids) {
         if (a.H % PQ_CH == 0 && ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.router & 15) == 0) {
             const int64_t tiles = (int64_t)((a.T + 31) / 32) * ((a.E + 31) / 32);
             if (tiles >= PQ_TILES)
@@ -573,14 +575,13 @@ int launch_prefill_route(const PrefillArgs& a, const int32_t* forced_ids, const 
         } else
             hipLaunchKernelGGL(k_pf_router, dim3((a.T + PR_T - 1) / PR_T, (a.E + PR_E - 1) / PR_E), dim3(256), 0, s, a.x,
                                a.router, a.H, a.T, a.E, a.logits);
-        hipLaunchKernelGGL(k_pf_topk, dim3((a.T + WAVES - 1) / WAVES), dim3(256), 0, s, a.logits, a.T, a.E, a.K, a.ids,
-                           a.w, a.hits, a.status);
     }
-    hipLaunchKernelGGL(k_pf_xpack, dim3(a.T), dim3(256), 0, s, a.x, a.H, a.x16, a.xexp);
-    hipLaunchKernelGGL(k_pf_group, dim3(1), dim3(1024), 0, s, a.ids, a.T, a.K, a.E, a.has_shared, a.pass_m, a.offsets,
-                       a.sorted, a.passes, a.pass_count, a.xexp);
-    if (a.has_shared && a.sh_gate_inp)
-        hipLaunchKernelGGL(k_pf_shgate, dim3(a.T), dim3(256), 0, s, a.x, a.sh_gate_inp, a.H, a.sg);
+    hipLaunchKernelGGL(k_pf_tokens, dim3(a.T), dim3(256), 0, s, a.x, a.H, a.x16, a.xexp,
+                       a.has_shared ? a.sh_gate_inp : nullptr, a.sg, forced_ids ? nullptr : a.logits, forced_ids, forced_w,
+                       a.E, a.K, a.ids, a.w, a.status);
+    const uint32_t kmul = (uint32_t)(((1ull << 32) + a.K - 1) / a.K);       // (0 for K = 1)
+    hipLaunchKernelGGL(k_pf_group, dim3(1), dim3(1024), 0, s, a.ids, a.T, a.K, kmul, a.E, a.has_shared, a.pass_m, a.offsets,
+                       a.sorted, a.passes, a.pass_count, a.xexp, a.hits);
     return (int)hipGetLastError();
 }
 
