@@ -5,8 +5,8 @@
 //
 // One workgroup of 8 waves per CU, or two of 4 (gm_waves), work through a
 // static list of items: item j of a launch is (pass, block of matrix rows),
-// and workgroup b takes items k, k + grid, k + 2 grid, ... with k =
-// pf_item_slot(b) (the row blocks of a pass on workgroups of one XCD).
+// and workgroup b takes one of every round of `grid` items: pf_item_slot (the
+// row blocks of a pass on workgroups of one XCD), pf_item_slot_full.
 //
 // The matrix columns are cut into slices, one per wave (groups of waves when
 // there are fewer slices than waves: each group then takes its own 16-row tiles).
@@ -190,6 +190,17 @@ WM_HD int pf_item_slot(int b, int grid, int R) {
     if (R <= 0 || grid % (PF_XCDS * R)) return b;
     const int x = b % PF_XCDS, q = b / PF_XCDS;
     return ((q / R) * PF_XCDS + x) * R + q % R;
+}
+
+// With passes of 32 pairs (busy experts of several passes), in a round that
+// every workgroup has an item of, an XCD takes a contiguous run of them: the
+// passes of an expert then read its rows from that XCD's L2.  4096 tokens
+// top-10, Q8_0 (80 pairs per expert): 3631 -> 3541 us per batch, 1001 tokens,
+// 64 experts 182.5 -> 179.1.  Passes of 16 keep the spread order (512 tokens
+// Q8_0 1374, in runs 1377; Q4_K 940, 936), as does the last, partial round
+// (1001 tokens in runs there too: 205).
+WM_HD int pf_item_slot_full(int b, int grid) {
+    return grid % PF_XCDS ? b : (b % PF_XCDS) * (grid / PF_XCDS) + b / PF_XCDS;
 }
 
 // Raw buffer resource over [p, p + bytes) (gfx9 word 3: 32-bit data format).
@@ -556,21 +567,25 @@ WM_DEV f32x4 mfma16(f16x8 a, f16x8 b, f32x4 c) { return __builtin_amdgcn_mfma_f3
 // reads; M: pairs per pass; NSB: 256-column super-blocks per ring slot.
 //
 // The items of one launch list (n_r routed ones, then the shared ones, up to
-// n_items) that this workgroup takes: k0, k0 + grid, ...
+// n_items) that this workgroup takes.  The list begins at position lo of the
+// launch's `total`, R row blocks per pass.
 #if defined(__HIP_DEVICE_COMPILE__)      // (buffer resources are device types)
 template <int AHL, int WT, int M, int NSB, int CW>
-WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int k0) {
+WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int lo, int total, int R) {
     typedef GmGeo<AHL, WT, M, NSB, CW> G;
     typedef KqRow<WT> F;
     constexpr int S = G::S, MT = G::MT, NI = G::NI, MSL = G::MSL, NSUB = G::NSUB;
     extern __shared__ __attribute__((aligned(16))) uint8_t gsm[];
     // the wave index is uniform: readfirstlane lets the compiler keep what depends on it in SGPRs
     const int tid = threadIdx.x, lane = tid & 63, wave = __builtin_amdgcn_readfirstlane(tid >> 6), g = lane >> 4, c = lane & 15;
-    if (k0 >= n_items) return;
+    const int grid = (int)gridDim.x, full = total / grid;
+    const int kl = pf_item_slot((int)blockIdx.x, grid, R), kf = M == 32 ? pf_item_slot_full((int)blockIdx.x, grid) : kl;
+    int i0 = lo / grid;
+    if (i0 * grid + (i0 < full ? kf : kl) < lo) ++i0;
 
     // item i of this workgroup: pass, first matrix row
     auto item = [&](int i, int& pass, int& row) __attribute__((always_inline)) -> bool {
-        const int j = k0 + i * (int)gridDim.x;
+        const int q = i0 + i, j = q * grid + (q < full ? kf : kl) - lo;
         if (j >= n_items) return false;
         if (j < n_r) {
             pass = j / a.nrb_r;
@@ -881,7 +896,7 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int k
         }
     };
 
-    item(0, cp, crow);
+    if (!item(0, cp, crow)) return;
     load_rec(cp, cur);
     setup_issue(expert_of(cp));
     for (int s = 0; s < S && iok; s++) issue_next();
@@ -961,8 +976,8 @@ template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB, int CW = 8>
 __global__ __launch_bounds__(64 * CW, 2) void k_pf_gemm(PfGemm a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const int n_rp = a.npass[0], n_r = a.sel == 2 ? 0 : n_rp * a.nrb_r;
-    pf_gemm_items<AHL, WT, M, NSB, CW>(a, n_rp, n_r, n_r + (a.sel == 1 ? 0 : a.npass[1] * a.nrb_s),
-                                       pf_item_slot((int)blockIdx.x, (int)gridDim.x, a.sel == 2 ? a.nrb_s : a.nrb_r));
+    const int n = n_r + (a.sel == 1 ? 0 : a.npass[1] * a.nrb_s);
+    pf_gemm_items<AHL, WT, M, NSB, CW>(a, n_rp, n_r, n, 0, n, a.sel == 2 ? a.nrb_s : a.nrb_r);
 #endif
 }
 
@@ -976,12 +991,10 @@ __global__ __launch_bounds__(64 * CW, 2) void k_pf_gemm(PfGemm a) {
 template <int AHL, int WT, int M, int NSB, int SWT, int CW>
 __global__ __launch_bounds__(64 * CW, 2) void k_pf_gemm2(PfGemm r, PfGemm s) {
 #if defined(__HIP_DEVICE_COMPILE__)
-    const int n_rp = r.npass[0], n_r = n_rp * r.nrb_r, grid = (int)gridDim.x;
-    const int k0 = pf_item_slot((int)blockIdx.x, grid, r.nrb_r);
-    pf_gemm_items<AHL, WT, M, NSB, CW>(r, n_rp, n_r, n_r, k0);
+    const int n_rp = r.npass[0], n_r = n_rp * r.nrb_r, n_s = s.npass[1] * s.nrb_s;
+    pf_gemm_items<AHL, WT, M, NSB, CW>(r, n_rp, n_r, n_r, 0, n_r + n_s, r.nrb_r);
     __syncthreads();                             // the ring and the staging change hands
-    const int first = k0 - n_r % grid;
-    pf_gemm_items<AHL, SWT, M, 1, CW>(s, n_rp, 0, s.npass[1] * s.nrb_s, first < 0 ? first + grid : first);
+    pf_gemm_items<AHL, SWT, M, 1, CW>(s, n_rp, 0, n_s, n_r, n_r + n_s, r.nrb_r);
 #endif
 }
 

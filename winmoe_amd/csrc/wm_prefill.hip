@@ -310,13 +310,14 @@ constexpr int PG_REG = 8, PG_SORT = 45056, PG_XEXP = 8192, PG_MAP = 4096;
 // cut into pass records of at most pm pairs (16 or 32): routed passes first,
 // in expert order, then the shared expert's; pass_count = {routed passes,
 // shared passes}.  A record also carries the x scale of each pair's token.
-// The experts' hit counters are raised here, by one add per expert: 4004
-// pairs over 64 experts spent 10 us on device atomics to 64 words.
+// The experts' hit counters are raised here, one add per expert: with an
+// atomic add per pair the top-K launch of 1001 tokens over 64 experts took
+// 17 us, the launch that holds its work now 7.
 //
 // Bound by latency: one workgroup, so the records are written by 8 threads
 // each (16-byte pieces of a pass side by side), a pair's token is a multiply
 // by kmul = ceil(2^32 / K) instead of a division, and ids are read PG_REG to
-// a thread at a time.
+// a thread at a time: 512 tokens top-10 23 -> 11 us, 4096 tokens 114 -> 27.
 __global__ __launch_bounds__(1024) void k_pf_group(const int32_t* __restrict__ ids, int T, int K, uint32_t kmul, int E,
                                                    int has_shared, int pm, int32_t* __restrict__ offsets,
                                                    int32_t* __restrict__ sorted, int32_t* __restrict__ passes,
