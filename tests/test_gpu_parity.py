@@ -780,6 +780,42 @@ def test_prefill_kquant_matches_oracle(wm, orc, gu, dn, sh, H):
     assert sl.layer.prefill_status() == 0
 
 
+@pytest.mark.parametrize("I,flag", [(256, 32), (512, 64), (4096, 32)])
+def test_prefill_q6k_small_scales_keep_precision(wm, orc, I, flag):
+    """Q6_K super-blocks of small negative scales (no quantiser makes them; a
+    file may hold them) lose nothing to the split of the scale: the products
+    with scales 1 and -1 are the same numbers but for the sign, so negating
+    the scales of down (or of up) negates the output.  A split that writes -1
+    as -16 + 15 adds two sums 16 and 15 times as large that cancel.  Bound:
+    the scale multiplies the sums of 128 columns (up: 256), 8 accumulations
+    of the matrix unit (4 units, hi and lo; up: 8 units), each off by at most
+    one unit in the last place, 2^-23 of the running sum, which grows with
+    the square root of its terms: sum_k sqrt(k / 8) 2^-23 = 5.6 * 2^-23, if
+    every rounding went one way.  One token against the oracle."""
+    from winmoe_amd import synth
+    E, K, H, T = 8, 2, 512, 40
+    cfg = synth.LayerConfig(f"pf_q6s_{I}", E=E, K=K, H=H, I=I, types=(Q6_K, Q6_K, Q6_K), tokens=1, routing="zipf",
+                            x_dtype="bf16", seed=21)
+    sl = synth.build_layer(cfg, max_tokens=T)
+    X = synth.make_hidden(cfg, tokens=T)
+    ids, w = _kq_routes(T, E, K, np.random.default_rng(I))
+    scales = [m.view(-1, 210)[:, 192:208] for m in (sl.gate, sl.up, sl.down)]
+    for f in scales:
+        f.fill_(1)
+    case(f"prefill q6k small scales I={I} flag={flag}")
+    pos = _prefill_flags(sl, X, ids, w, flag)
+    assert np.isfinite(pos).all() and np.abs(pos).max() > 0
+    for name, f in (("down", scales[2]), ("up", scales[1])):
+        f.fill_(255)                                   # int8 -1
+        case(f"prefill q6k small scales I={I} flag={flag} {name} negated")
+        neg = _prefill_flags(sl, X, ids, w, flag)
+        f.fill_(1)
+        print(f"{name}: {rel_l2(-neg, pos):.2e}", flush=True)
+        assert rel_l2(-neg, pos) <= 5.6 * 2.0 ** -23, (name, rel_l2(-neg, pos))
+        _, _, ref = oracle_token(orc, sl, host(X[3].float()), ids=ids[3], w=w[3])
+        assert rel_l2(-neg[3], ref) <= LAYER_TOL
+
+
 @pytest.mark.parametrize("name", ["c3", "c4"])
 def test_prefill_kquant_full_layer(wm, orc, name):
     """A 512-token prefill through the full 512-expert layer of the Q4_K /

@@ -43,7 +43,8 @@
 //     are a second MFMA of the activations with the replicated min, times
 //     dmin;
 //   * Q6_K (q6k_dequant.h:112-141): q times its int8 scale needs 13 bits, so
-//     the scale is split into 16 s1 + s0 and each part multiplies q exactly.
+//     the scale is split into 16 s1 + s0, s1 the nearest (a scale of -7 .. 7
+//     is s0 alone), and each part multiplies q exactly.
 // Down activations carry a power-of-two scale per (pair, 128 columns), which
 // multiplies the sum of those columns.
 #pragma once
@@ -350,7 +351,10 @@ template <> struct KqRow<Q5_K> : Kq45<5> {};     // q5k_dequant.h:19-25, 98-131
 // 32 (j & 1) + l] (low nibble for j < 2, high else), qh[32 h + l] bits 2 j.
 // This lane: ql bytes 64 h + 16 g .. + 15 (j & 1 = g / 2, l = 16 (g & 1) ..):
 // low nibbles in sub-block 8 h + g, high nibbles in 8 h + 4 + g.  scale = 16
-// s1 + s0: unit(h, u, 1) = q s1, unit(h, u, 0) = q s0, both exact.
+// s1 + s0 with s0 in [-8, 7]: unit(h, u, 1) = q s1, unit(h, u, 0) = q s0, both
+// exact, and 16 |s1| <= |scale| + 8, so that the two sums do not cancel (with
+// s0 in [0, 15] a scale of -1 is -16 + 15: rows of such scales then missed the
+// negative of the rows with scale 1 by 2.3e-6; now by 3 to 6e-8).
 template <> struct KqRow<Q6_K> {
     static constexpr int AL = 2;
     static constexpr bool FOLD = false, MINS = false;
@@ -379,7 +383,7 @@ template <> struct KqRow<Q6_K> {
         for (int n = 0; n < 2; n++)
 #pragma unroll
             for (int part = 0; part < 2; part++) {
-                const int s = sb[2 * h + n], v = part ? s >> 4 : s & 15;
+                const int s = sb[2 * h + n], s1 = (s + 8) >> 4, v = part ? s1 : s - 16 * s1;
                 f16x2 f = h2((float)v);
                 c2[n][part] = f * h2(-1056.0f);              // 1024 + 32 (values q + 32), |v| <= 15: exact
                 s2[n][part] = n ? f * h2(0.0625f) : f;
