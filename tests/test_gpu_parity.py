@@ -612,6 +612,46 @@ def test_prefill_grouping_limits(wm, T, K, E):
     assert np.array_equal(part.view(np.uint32), whole[pick].view(np.uint32))
 
 
+@pytest.mark.parametrize("I,Is,flag,want", [(512, 0, 32, [16, 16]), (512, 0, 64, [32, 32]), (2048, 0, 64, [32, 32]),
+                                            (4096, 0, 32, [16, 16]), (4096, 0, 64, [32, 16]),
+                                            (4096, 4096, 64, [32, 16]), (512, 4096, 64, [32, 16, 16]), (4096, 0, 0, [32, 16])])
+def test_prefill_pass_flags_are_obeyed(wm, orc, I, Is, flag, want):
+    """The forced pass size (or, at 17 pairs per expert, the default 32) is the
+    one the GEMMs run with (read from the names of the launched kernels, gate/up
+    then down), also where down has registers
+    for 16 pairs only (I above 2048) and the pairs are grouped again for it:
+    expert 0 with passes of 32, 32 and 6, a second call the same, hit counters
+    raised once a call, one token against the oracle."""
+    import ctypes as C
+    import re
+    import torch
+    from torch.profiler import ProfilerActivity, profile
+    from winmoe_amd import synth
+    E, K, H, T = 8, 2, 512, 70
+    cfg = synth.LayerConfig(f"pf_flag_{I}_{Is}", E=E, K=K, H=H, I=I, types=(Q8_0, Q8_0, Q8_0),
+                            shared_types=(Q8_0,) * 3 if Is else None, shared_inter=Is, shared_gate_inp=bool(Is), tokens=1,
+                            routing="zipf", x_dtype="bf16", seed=23)
+    sl = synth.build_layer(cfg, max_tokens=T)
+    X = synth.make_hidden(cfg, tokens=T)
+    ids, w = _kq_routes(T, E, K, np.random.default_rng(I + Is))
+    case(f"prefill pass flags I={I} shared={Is} flag={flag}")
+    first = _prefill_flags(sl, X, ids, w, flag)
+    with profile(activities=[ProfilerActivity.CUDA]) as p:
+        out = _prefill_flags(sl, X, ids, w, flag)
+        torch.cuda.synchronize()
+    ev = sorted((e for e in p.events() if "k_pf_gemm<" in e.name), key=lambda e: e.time_range.start)
+    got = [int(re.search(r"<([\d, ]+)>", e.name).group(1).split(",")[-3]) for e in ev]     # <.., pairs, super-blocks, waves>
+    assert got == want, [e.name for e in ev]
+    assert np.array_equal(out.view(np.uint32), first.view(np.uint32))
+    off = [C.c_int64() for _ in range(3)]
+    wm.load().wm_prefill_workspace_routing(C.byref(sl.layer.desc), sl.layer.pf_tokens, *[C.byref(o) for o in off])
+    o = off[2].value
+    hits = host(sl.layer.pf_ws[o:o + 4 * E].view(torch.int32))
+    assert np.array_equal(hits, 2 * np.bincount(ids.ravel(), minlength=E))
+    _, _, ref = oracle_token(orc, sl, host(X[69].float()), ids=ids[69], w=w[69])
+    assert rel_l2(out[69], ref) <= LAYER_TOL
+
+
 def test_prefill_rejects_unsupported_widths(wm):
     """Prefill needs H, I and the shared width to be multiples of 256."""
     from winmoe_amd import synth

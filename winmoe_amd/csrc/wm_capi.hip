@@ -996,7 +996,7 @@ static int run_prefill(const wm_layer_desc* d, const uint16_t* x, int T, const i
     hipStream_t s = S(stream);
     uint8_t* w8 = (uint8_t*)ws;
     PrefillArgs a = {};
-    a.H = d->hidden; a.I = d->inter; a.Is = Ishared(d); a.E = d->n_experts; a.K = d->top_k; a.T = T;
+    a.H = d->hidden; a.I = d->inter; a.Is = sh ? Ishared(d) : 0; a.E = d->n_experts; a.K = d->top_k; a.T = T;
     a.has_shared = sh ? 1 : 0;
     a.gt = d->gate_type; a.dt = d->down_type;
     a.sgt = sh ? d->sh_gate_type : a.gt; a.sdt = sh ? d->sh_down_type : a.dt;
@@ -1019,8 +1019,7 @@ static int run_prefill(const wm_layer_desc* d, const uint16_t* x, int T, const i
                  (WM_FLAG_PREFILL_PASS16 | WM_FLAG_PREFILL_PASS32));
     a.pass_m = (d->flags & WM_FLAG_PREFILL_PASS16)   ? 16
                : (d->flags & WM_FLAG_PREFILL_PASS32) ? 32
-                                                     : prefill_pass_size(T, a.K, a.E, a.gt);
-    if (std::max(a.I, sh ? a.Is : 0) > 2048) a.pass_m = 16;     // down holds no more than 16 pairs of longer rows
+                                                     : prefill_pass_size(T, a.K, a.E, a.gt, prefill_wide(a.I, a.Is));
     // the expert GEMMs read 16-byte granules from row starts
     WM_CHECK_ARG(al(a.gate, 16) && al(a.up, 16) && al(a.down, 16) && a.gstride % 16 == 0 && a.ustride % 16 == 0 &&
                  a.dstride % 16 == 0 && (!sh || (al(a.sh_gate, 16) && al(a.sh_up, 16) && al(a.sh_down, 16))));

@@ -11,7 +11,7 @@ namespace wm {
 // A (token, slot) pair p = t * K + k is one routed use of an expert; pair
 // T * K + t is token t's use of the shared expert.
 struct PrefillArgs {
-    int32_t H, I, Is, E, K, T, has_shared;
+    int32_t H, I, Is, E, K, T, has_shared;      // Is: 0 without a shared expert
     int32_t gt, dt, sgt, sdt;   // weight formats: routed gate = up, down; shared gate = up, down
     const uint16_t* x;          // bf16 [T][H]
     const float* router;        // fp32 [E][H]
@@ -55,8 +55,14 @@ inline int64_t prefill_max_passes(int64_t T, int64_t K, int64_t E) { return (T *
 // with Zipf routing over 512 experts (ms per batch, 16 / 32): Q8_0 at 10
 // pairs per expert 1.54 / 1.56, at 20 2.16 / 1.80; Q4_K gate/up, Q6_K down
 // at 3 pairs 1.45 / 1.54, at 12 2.14 / 1.95.
-inline int prefill_pass_size(int64_t T, int64_t K, int64_t E, int gate_type) {
-    return T * K <= (gate_type == Q8_0 ? 10 : 4) * E ? 16 : 32;
+// Wide rows (prefill_wide: only gate/up can take passes of 32, and the pairs
+// are grouped twice): K-quants from 16 pairs on.  us per batch, 16 / 32, 64
+// experts, I 4096: Q4_K, Q6_K, H 4096 at 6 pairs 572 / 647, at 16 769 / 762, at
+// 40 1465 / 1333; Q2_K, Q3_K, H 2048 at 12 331 / 350, at 16 363 / 360, at 28 557
+// / 508; Q8_0, H 2048 at 6 397 / 413, at 9 426 / 416, at 20 561 / 500.
+inline bool prefill_wide(int64_t I, int64_t Is) { return I > 2048 || Is > 2048; }
+inline int prefill_pass_size(int64_t T, int64_t K, int64_t E, int gate_type, bool wide) {
+    return T * K <= (gate_type == Q8_0 ? 10 : wide ? 16 : 4) * E ? 16 : 32;
 }
 
 // Weight formats the expert GEMMs read: gate and up (one format for both) and down.

@@ -310,9 +310,9 @@ constexpr int PG_REG = 8, PG_SORT = 45056, PG_XEXP = 8192, PG_MAP = 4096;
 // cut into pass records of at most pm pairs (16 or 32): routed passes first,
 // in expert order, then the shared expert's; pass_count = {routed passes,
 // shared passes}.  A record also carries the x scale of each pair's token.
-// The experts' hit counters are raised here, one add per expert: with an
-// atomic add per pair the top-K launch of 1001 tokens over 64 experts took
-// 17 us, the launch that holds its work now 7.
+// The experts' hit counters are raised here (hits not NULL), one add per
+// expert: with an atomic add per pair the top-K launch of 1001 tokens over 64
+// experts took 17 us, the launch that holds its work now 7.
 //
 // Bound by latency: one workgroup, so the records are written by 8 threads
 // each (16-byte pieces of a pass side by side), a pair's token is a multiply
@@ -360,7 +360,7 @@ __global__ __launch_bounds__(1024) void k_pf_group(const int32_t* __restrict__ i
     for (int base = 0; base < G; base += 1024) {
         const int e = base + tid;
         const int n = e < G ? cnt[e] : 0;
-        if (e < E && n) hits[e] += (uint32_t)n;
+        if (e < E && n && hits) hits[e] += (uint32_t)n;
         int2 tot;
         const int2 ex = block_excl_scan2(make_int2(n, (n + pm - 1) / pm), wsum, &tot);
         if (e < G) {
@@ -563,6 +563,12 @@ __global__ __launch_bounds__(256) void k_pf_combine(PrefillArgs a) {
 
 // ------------------------------------------------------------------ launcher
 
+static void launch_group(const PrefillArgs& a, uint32_t* hits, hipStream_t s) {
+    const uint32_t kmul = (uint32_t)(((1ull << 32) + a.K - 1) / a.K);       // (0 for K = 1)
+    hipLaunchKernelGGL(k_pf_group, dim3(1), dim3(1024), 0, s, a.ids, a.T, a.K, kmul, a.E, a.has_shared, a.pass_m, a.offsets,
+                       a.sorted, a.passes, a.pass_count, a.xexp, hits);
+}
+
 int launch_prefill_route(const PrefillArgs& a, const int32_t* forced_ids, const float* forced_w, hipStream_t s) {
     if (!forced_ids) {
         if (a.H % PQ_CH == 0 && ((uintptr_t)a.x & 15) == 0 && ((uintptr_t)a.router & 15) == 0) {
@@ -580,9 +586,7 @@ int launch_prefill_route(const PrefillArgs& a, const int32_t* forced_ids, const 
     hipLaunchKernelGGL(k_pf_tokens, dim3(a.T), dim3(256), 0, s, a.x, a.H, a.x16, a.xexp,
                        a.has_shared ? a.sh_gate_inp : nullptr, a.sg, forced_ids ? nullptr : a.logits, forced_ids, forced_w,
                        a.E, a.K, a.ids, a.w, a.status);
-    const uint32_t kmul = (uint32_t)(((1ull << 32) + a.K - 1) / a.K);       // (0 for K = 1)
-    hipLaunchKernelGGL(k_pf_group, dim3(1), dim3(1024), 0, s, a.ids, a.T, a.K, kmul, a.E, a.has_shared, a.pass_m, a.offsets,
-                       a.sorted, a.passes, a.pass_count, a.xexp, a.hits);
+    launch_group(a, a.hits, s);
     return (int)hipGetLastError();
 }
 
@@ -652,7 +656,17 @@ static int down_rows(const PrefillArgs& a) {
     return a.H % 512 || items < 2 * grid ? (2 * items < grid ? 128 : 256) : 512;
 }
 
-int launch_prefill_down(const PrefillArgs& a, hipStream_t s) {
+// Down of rows longer than 2048 columns (slices of 512, hi and lo) has
+// registers for 16 pairs only: after gate/up in passes of 32 the pairs are
+// grouped again.  That launch is 10 us; gate/up in passes of 16 as well cost a
+// busy expert more: 1500 tokens top-2 of 8 experts, H and I 4096, Q8_0, gate/up
+// 925 us in passes of 16, 721 in passes of 32.
+int launch_prefill_down(const PrefillArgs& args, hipStream_t s) {
+    PrefillArgs a = args;
+    if (a.pass_m > 16 && prefill_wide(a.I, a.Is)) {
+        a.pass_m = 16;
+        launch_group(a, nullptr, s);
+    }
     PfGemm g = {};
     g.w0 = a.down; g.w1 = a.down; g.st0 = g.st1 = a.dstride;
     g.s0 = g.s1 = a.sh_down;
