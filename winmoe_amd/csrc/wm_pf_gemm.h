@@ -351,7 +351,7 @@ template <> struct KqRow<Q5_K> : Kq45<5> {};     // q5k_dequant.h:19-25, 98-131
 // 32 (j & 1) + l] (low nibble for j < 2, high else), qh[32 h + l] bits 2 j.
 // This lane: ql bytes 64 h + 16 g .. + 15 (j & 1 = g / 2, l = 16 (g & 1) ..):
 // low nibbles in sub-block 8 h + g, high nibbles in 8 h + 4 + g.  scale = 16
-// s1 + s0 with s0 in [-8, 7]: unit(h, u, 1) = q s1, unit(h, u, 0) = q s0, both
+// s1 + s0 with s0 in [-8, 8]: unit(h, u, 1) = q s1, unit(h, u, 0) = q s0, both
 // exact, and 16 |s1| <= |scale| + 8, so that the two sums do not cancel (with
 // s0 in [0, 15] a scale of -1 is -16 + 15: rows of such scales then missed the
 // negative of the rows with scale 1 by 2.3e-6; now by 3 to 6e-8).
@@ -380,15 +380,18 @@ template <> struct KqRow<Q6_K> {
     }
     WM_DEV void half(int h) {
 #pragma unroll
-        for (int n = 0; n < 2; n++)
+        for (int n = 0; n < 2; n++) {
+            // s1 = the scale / 16 rounded (fp16 holds the integers around 1536 and no fractions), s0 the rest in [-8, 8]
+            const _Float16 sv = (_Float16)(int16_t)sb[2 * h + n];
+            const f16x2 s = {sv, sv}, s1 = fma2(s, h2(0.0625f), h2(1536.0f)) - h2(1536.0f), s0 = fma2(s1, h2(-16.0f), s);
 #pragma unroll
             for (int part = 0; part < 2; part++) {
-                const int s = sb[2 * h + n], s1 = (s + 8) >> 4, v = part ? s1 : s - 16 * s1;
-                f16x2 f = h2((float)v);
-                c2[n][part] = f * h2(-1056.0f);              // 1024 + 32 (values q + 32), |v| <= 15: exact
+                const f16x2 f = part ? s1 : s0;
                 s2[n][part] = n ? f * h2(0.0625f) : f;
-                if (n) c2[n][part] = f * h2(-96.0f);         // (1024 + 16 * 32) / 16
+                // 1024 + 32 (values q + 32), or (1024 + 16 * 32) / 16; |f| <= 8: exact
+                c2[n][part] = n ? f * h2(-96.0f) : f * h2(-1056.0f);
             }
+        }
     }
     // the 8 values as 1024 + (q + 32) (low nibbles) or 1024 + 16 (q + 32)
     WM_DEV void raw(int h, int u, uint32_t k64, f16x2* v) const {
