@@ -652,6 +652,36 @@ def test_prefill_pass_flags_are_obeyed(wm, orc, I, Is, flag, want):
     assert rel_l2(out[69], ref) <= LAYER_TOL
 
 
+@pytest.mark.parametrize("H,I,types", [(4096, 256, (Q8_0, Q8_0, Q8_0)), (512, 2048, (Q8_0, Q8_0, Q8_0)),
+                                       (512, 1024, (Q2_K, Q2_K, Q6_K)), (4096, 2048, (Q4_K, Q4_K, Q5_K)),
+                                       (256, 512, (Q3_K, Q3_K, Q4_K)), (2048, 256, (Q6_K, Q6_K, Q2_K)),
+                                       (1024, 1024, (Q5_K, Q5_K, Q3_K))])
+def test_prefill_row_tiles(wm, orc, H, I, types):
+    """Passes of 32 leave their second row tile out at 16 pairs or fewer:
+    experts of 1, 15, 16, 17, 31, 32, 33, 48 and 49 pairs in one launch (items
+    of both kinds follow each other in a workgroup) give the bits of passes of
+    16, where every tile is its own pass; one token of every expert against
+    the oracle."""
+    from winmoe_amd import synth
+    counts = [1, 15, 16, 17, 31, 32, 33, 48, 49]
+    E, T = len(counts), sum(counts)
+    cfg = synth.LayerConfig(f"pf_tiles_{H}_{I}_{types[0]}", E=E, K=1, H=H, I=I, types=types, tokens=1, routing="zipf",
+                            x_dtype="bf16", seed=27)
+    sl = synth.build_layer(cfg, max_tokens=T)
+    X = synth.make_hidden(cfg, tokens=T)
+    rng = np.random.default_rng(H + I)
+    ids = rng.permutation(np.repeat(np.arange(E), counts)).astype(np.int32).reshape(T, 1)
+    w = rng.random((T, 1)).astype(np.float32)
+    case(f"prefill row tiles H={H} I={I} types={types}")
+    out = _prefill_flags(sl, X, ids, w, wm._lib.FLAG_PREFILL_PASS32)
+    assert np.isfinite(out).all()
+    _check_pass_sizes(sl, X, ids, w, out)
+    for e in range(E):
+        t = int(np.flatnonzero(ids[:, 0] == e)[-1])
+        _, _, ref = oracle_token(orc, sl, host(X[t].float()), ids=ids[t], w=w[t])
+        assert rel_l2(out[t], ref) <= LAYER_TOL, (e, rel_l2(out[t], ref))
+
+
 def test_prefill_rejects_unsupported_widths(wm):
     """Prefill needs H, I and the shared width to be multiples of 256."""
     from winmoe_amd import synth

@@ -282,7 +282,15 @@ WM_DEV f16x8 rep4(f16x2 a) { return cat4(a, a, a, a); }
 // holds exactly) and mins(u) the sub-block min; the weight is
 // d * unit - dmin * mins.  Values are decoded as (1024 + 2^k q) * (sc / 2^k)
 // - 1024 * sc / 2^k, one rounding of an exact result.
+// pin(): the loaded registers become unknown to the compiler, so that it does
+// not decode ahead of a branch what both sides need (the decoded values of all
+// units at once: up to 240 registers in scratch).
 template <int WT> struct KqRow;
+
+template <int N> WM_DEV void pin_dw(uint32_t (&w)[N]) {
+#pragma unroll
+    for (int i = 0; i < N; i++) asm volatile("" : "+v"(w[i]));
+}
 
 // Q4_K and Q5_K: half h is qs bytes 64 h .. + 63, low nibbles columns 32 i +
 // l of byte 32 i + l, high nibbles 32 columns on.  This lane: bytes 16 g ..
@@ -303,6 +311,17 @@ template <int BITS> struct Kq45 {
         if constexpr (BITS == 5) ld_dw<16, 4>(slot, o + 16 + 16 * (g & 1), qh);
         ld_dw<16, 4>(slot, o + (BITS == 5 ? 48 : 16) + 16 * g, q[0]);
         ld_dw<16, 4>(slot, o + (BITS == 5 ? 48 : 16) + 64 + 16 * g, q[1]);
+    }
+    WM_DEV void pin() {
+#pragma unroll
+        for (int i = 0; i < 4; i++) {
+            uint32_t v = hd[i];
+            asm volatile("" : "+v"(v));
+            hd[i] = v;
+        }
+        if constexpr (BITS == 5) pin_dw(qh);
+        pin_dw(q[0]);
+        pin_dw(q[1]);
     }
     WM_DEV void head(int g) {
         d = h2f(hd[0]);
@@ -374,6 +393,16 @@ template <> struct KqRow<Q6_K> {
         for (int i = 0; i < 4; i++) sb[i] = *(const int8_t*)(slot + o + 192 + 4 * i + g);
         d16 = *(const uint16_t*)(slot + o + 208);
     }
+    WM_DEV void pin() {
+#pragma unroll
+        for (int h = 0; h < 2; h++) {
+            pin_dw(ql[h]);
+            pin_dw(qh[h]);
+        }
+#pragma unroll
+        for (int i = 0; i < 4; i++) asm volatile("" : "+v"(sb[i]));
+        asm volatile("" : "+v"(d16));
+    }
     WM_DEV void head(int g) {
         d = h2f(d16);
         sh = 4 - 2 * (g >> 1);
@@ -432,6 +461,13 @@ template <> struct KqRow<Q3_K> {                 // hmask[32] qs[64] scales[12] 
         ld_dw<AL, 3>(slot, o + 96, s3);
         d16 = *(const uint16_t*)(slot + o + 108);
     }
+    WM_DEV void pin() {
+        pin_dw(hm);
+        pin_dw(q[0]);
+        pin_dw(q[1]);
+        pin_dw(s3);
+        asm volatile("" : "+v"(d16));
+    }
     WM_DEV void head(int g) {
         d = h2f(d16);
         dmin = 0.0f;
@@ -482,6 +518,12 @@ template <> struct KqRow<Q2_K> {                 // scales[16] qs[64] d dmin
         ld_dw<AL, 2>(slot, o + 48 + 8 * g, q[1]);
         ld_dw<AL, 1>(slot, o + 80, &dd);
     }
+    WM_DEV void pin() {
+        pin_dw(sb);
+        pin_dw(q[0]);
+        pin_dw(q[1]);
+        asm volatile("" : "+v"(dd));
+    }
     WM_DEV void head(int g) {
         d = h2f(dd);
         dmin = h2f(dd >> 16);
@@ -531,6 +573,9 @@ template <> struct KqRow<Q8_0> {
             d16[b] = *(const uint16_t*)(slot + o + 34 * b);
         }
     }
+    // the decode is short: keeping only its start apart was faster (4096 tokens 3584 us per batch, with every
+    // register unknown 3627)
+    WM_DEV void pin() { asm volatile("" ::: "memory"); }
     WM_DEV float scale(int b) const { return h2f(d16[b]); }
     WM_DEV f16x8 unit(int b) const {
         const uint32_t K = 0x64646464u, X = 0x80808080u;
@@ -676,23 +721,16 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
     constexpr int NO = CW == 4 ? MT : 1;
     const int tmt = CW == 8 && MT == 2 ? tid >> 8 : 0, om = 16 * tmt + 4 * ((tid & 255) >> 6) + (tid & 3), orow = (tid >> 2) & 15;
     struct Rec {
-        int n, own[NO], xe[NO];        // pairs; this thread's output pairs and their x exponents
-        int pid[MT];                   // pair of operand row c
-        int4 pq[MT];                   // down: pairs of accumulator rows 4g .. 4g + 3
+        int n, xe[NO];                 // pairs; gate/up: the x exponents of this thread's output pairs
+        int pid[MT];                   // pair of operand row c (c = 4g + i: of accumulator row i)
     };
     auto load_rec = [&](int pass, Rec& r) __attribute__((always_inline)) {
         const int32_t* p = a.recs + (int64_t)pass * GM_REC;
         r.n = ((cint_t*)a.recs)[(int64_t)pass * GM_REC + 1];
 #pragma unroll
-        for (int q = 0; q < NO; q++) {
-            r.own[q] = p[4 + om + 16 * q];
-            r.xe[q] = G::GU ? (int)((const int8_t*)(p + 4 + GM_M))[om + 16 * q] : 0;
-        }
+        for (int q = 0; q < NO; q++) r.xe[q] = G::GU ? (int)((const int8_t*)(p + 4 + GM_M))[om + 16 * q] : 0;
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            r.pid[mt] = p[4 + 16 * mt + c];
-            if constexpr (!G::GU) r.pq[mt] = *(const int4*)(p + 4 + 16 * mt + 4 * g);
-        }
+        for (int mt = 0; mt < MT; mt++) r.pid[mt] = p[4 + 16 * mt + c];
     };
     u32x4 A[AHL][MT][MSL][8 * NSB];
     f32x4 asc[MT][G::GU ? 1 : MSL][G::GU ? 1 : 2 * NSB];
@@ -700,7 +738,13 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
     auto load_act = [&](const Rec& r) __attribute__((always_inline)) {
 #pragma unroll
         for (int mt = 0; mt < MT; mt++) {
+            if (mt && r.n <= 16) continue;
             const int64_t row = G::GU ? pair_token(r.pid[mt], a.T, a.K) : r.pid[mt];
+            int pr[4];                 // down: pairs of accumulator rows 4g .. 4g + 3
+            if constexpr (!G::GU) {
+#pragma unroll
+                for (int i = 0; i < 4; i++) pr[i] = __shfl(r.pid[mt], 4 * g + i);
+            }
 #pragma unroll
             for (int s = 0; s < MSL; s++) {
                 if (s && s >= ns) continue;
@@ -713,7 +757,6 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
                 }
                 if constexpr (!G::GU) {
                     const int k = (scol + s * G::KC) / 128;
-                    const int pr[4] = {r.pq[mt].x, r.pq[mt].y, r.pq[mt].z, r.pq[mt].w};
 #pragma unroll
                     for (int h = 0; h < 2 * NSB; h++)
 #pragma unroll
@@ -722,6 +765,9 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
             }
         }
     };
+    // the current pass fills its second row tile: a pass of 32 with 16 pairs or
+    // fewer leaves that tile's loads, products and sums out
+    bool two = false;
     // K-quant operands hold their 8 columns in the order 0 2 1 3 4 6 5 7
     auto order_act = [&]() __attribute__((always_inline)) {
         if constexpr (G::KQ) {
@@ -731,7 +777,7 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
                 for (int mt = 0; mt < MT; mt++)
 #pragma unroll
                     for (int s = 0; s < MSL; s++) {
-                        if (s && s >= ns) continue;
+                        if ((mt && !two) || (s && s >= ns)) continue;
 #pragma unroll
                         for (int b = 0; b < 8 * NSB; b++) {
                             const u32x4 v = A[h][mt][s][b];
@@ -744,42 +790,44 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
         }
     };
 
-    // ---- one ring slot: wait for it, take it into registers, refill it, add
-    // its products to acc
+    // ---- one ring slot: wait for it, take it into registers, refill it (take);
+    // add its products with the first MN row tiles of the pass to acc (sums)
     const f32x4 zero = {0.0f, 0.0f, 0.0f, 0.0f};
     const uint32_t k64 = opaque_e1024();
     const int rsh = (int)(((uint32_t)c * rb) & 15u);         // row c's start past a 16-byte boundary
     int cslot = 0;
-    auto slot = [&](auto s_tag, f32x4(&acc)[MT]) __attribute__((always_inline)) {
+    auto take = [&](auto s_tag, F(&row)[NSB]) __attribute__((always_inline)) {
         constexpr int SI = decltype(s_tag)::value;
         if (outst == S) WM_WAIT_VMCNT((S - 1) * NI);
         else WM_WAIT_VMCNT(0);
         asm volatile("" ::: "memory");
         const uint8_t* rowp = gsm + wave * (S * G::SLOT) + cslot * G::SLOT + c * G::RSLOT;
         const int o = F::AL >= 16 ? 0 : rsh + (((sl * ns + SI) * G::CHUNK) & 15);
-        F row[NSB];
 #pragma unroll
         for (int sb = 0; sb < NSB; sb++) row[sb].load(rowp, o + sb * (G::CHUNK / NSB), g);
         gm_wait_lds();
         --outst;
         cslot = cslot + 1 == S ? 0 : cslot + 1;
         if (iok) issue_next();
+    };
+    auto sums = [&](auto s_tag, auto m_tag, F(&row)[NSB], f32x4(&acc)[MT]) __attribute__((always_inline)) {
+        constexpr int SI = decltype(s_tag)::value, MN = decltype(m_tag)::value;
 #pragma unroll
         for (int sb = 0; sb < NSB; sb++) {
             F& f = row[sb];
             if constexpr (!G::KQ) {
-                f32x4 t[2][MT];
+                f32x4 t[2][MN];
 #pragma unroll
-                for (int mt = 0; mt < MT; mt++) t[0][mt] = t[1][mt] = zero;
+                for (int mt = 0; mt < MN; mt++) t[0][mt] = t[1][mt] = zero;
                 // the scaling of a block's products comes after the next
                 // block's MFMAs are sent, so that it does not wait for them
-                f32x4 P[2][MT];
+                f32x4 P[2][MN];
 #pragma unroll
                 for (int b = 0; b <= 8; b++) {
                     if (b < 8) {
                         const f16x8 B = f.unit(b);
 #pragma unroll
-                        for (int mt = 0; mt < MT; mt++) {
+                        for (int mt = 0; mt < MN; mt++) {
                             P[b & 1][mt] = mfma16(__builtin_bit_cast(f16x8, A[0][mt][SI][8 * sb + b]), B, zero);
                             if constexpr (AHL == 2)
                                 P[b & 1][mt] = mfma16(__builtin_bit_cast(f16x8, A[AHL - 1][mt][SI][8 * sb + b]), B, P[b & 1][mt]);
@@ -789,7 +837,7 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
                     if (b > 0) {
                         const float d = f.scale(b - 1);
 #pragma unroll
-                        for (int mt = 0; mt < MT; mt++) {
+                        for (int mt = 0; mt < MN; mt++) {
                             f32x4& r = G::GU ? acc[mt] : t[(b - 1) >> 2][mt];
 #pragma unroll
                             for (int i = 0; i < 4; i++) r[i] = fmaf(d, P[(b - 1) & 1][mt][i], r[i]);
@@ -798,7 +846,7 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
                 }
                 if constexpr (!G::GU) {
 #pragma unroll
-                    for (int mt = 0; mt < MT; mt++)
+                    for (int mt = 0; mt < MN; mt++)
 #pragma unroll
                         for (int h = 0; h < 2; h++)
 #pragma unroll
@@ -809,12 +857,12 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
                 // NQ sums: the products with q sc (Q6_K: with q s1 and q s0);
                 // the mins.  Gate/up: over the super-block, down: per half.
                 constexpr int NQ = F::FOLD ? 1 : 2;
-                f32x4 sq[NQ][MT], sm[MT];
+                f32x4 sq[NQ][MN], sm[MN];
 #pragma unroll
                 for (int h = 0; h < 2; h++) {
                     if (h == 0 || !G::GU) {
 #pragma unroll
-                        for (int mt = 0; mt < MT; mt++) {
+                        for (int mt = 0; mt < MN; mt++) {
 #pragma unroll
                             for (int k = 0; k < NQ; k++) sq[k][mt] = zero;
                             sm[mt] = zero;
@@ -834,7 +882,7 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
                             for (int k = 0; k < NQ; k++) B[k] = f.unit(v, u, k);
                         }
 #pragma unroll
-                        for (int mt = 0; mt < MT; mt++)
+                        for (int mt = 0; mt < MN; mt++)
 #pragma unroll
                             for (int l = 0; l < AHL; l++) {
                                 const f16x8 av = __builtin_bit_cast(f16x8, A[l][mt][SI][8 * sb + 4 * h + u]);
@@ -845,7 +893,7 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
                     }
                     if (h == 1 || !G::GU) {
 #pragma unroll
-                        for (int mt = 0; mt < MT; mt++) {
+                        for (int mt = 0; mt < MN; mt++) {
                             f32x4 r = G::GU ? acc[mt] : zero;
 #pragma unroll
                             for (int i = 0; i < 4; i++) {
@@ -861,15 +909,28 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
             }
         }
     };
+    auto slot = [&](auto s_tag, f32x4(&acc)[MT]) __attribute__((always_inline)) {
+        F row[NSB];
+        take(s_tag, row);
+        if constexpr (MT == 1) sums(s_tag, std::integral_constant<int, 1>{}, row, acc);
+        else if (two) sums(s_tag, std::integral_constant<int, 2>{}, row, acc);
+        else {
+#pragma unroll
+            for (int sb = 0; sb < NSB; sb++) row[sb].pin();
+            sums(s_tag, std::integral_constant<int, 1>{}, row, acc);
+        }
+    };
 
     // ---- a tile's partial sums, in slice order, to out(pair slot group, value)
     int pbuf = 0, ci = 0, cp = 0, crow = 0;
     Rec cur, nxt;
+    int own[NO];
     float* stg = (float*)(gsm + G::STG);
     auto finish = [&](int mat, int st, const f32x4(&acc)[MT]) __attribute__((always_inline)) {
         float* pb = (float*)(gsm + G::PBASE + pbuf * G::PART);
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) *(f32x4*)(pb + (wave * MT + mt) * 256 + 4 * lane) = acc[mt];
+        for (int mt = 0; mt < MT; mt++)
+            if (!mt || two) *(f32x4*)(pb + (wave * MT + mt) * 256 + 4 * lane) = acc[mt];
         gm_bar();
         pbuf ^= 1;
         // r: row group of this thread's q-th output
@@ -889,13 +950,14 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
                     *sp = silu_mul(*sp * xs, v * xs);
                 }
             } else {
-                if (om + 16 * q < cur.n) a.y[(int64_t)cur.own[q] * a.y_ld + crow + row] = v;
+                if (om + 16 * q < cur.n) a.y[(int64_t)own[q] * a.y_ld + crow + row] = v;
             }
         };
         if constexpr (CW == 4 || MT == 2) {
             for (int r = 0; r < nrg; r++)
 #pragma unroll
-                for (int q = 0; q < NO; q++) reduce(r, q);
+                for (int q = 0; q < NO; q++)
+                    if (!(tmt + q) || two) reduce(r, q);
         } else if (nrg == 1) {
             if ((tid >> 8) == (st & 1)) reduce(0, 0);        // 4 waves each, in turn
         } else {
@@ -913,15 +975,17 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
     if (nok) load_rec(np, nxt);
     else nxt = cur;
     for (;;) {
+        two = MT > 1 && cur.n > 16;
         order_act();
         // the next record is in (its loads are older than the activations' wait)
 #pragma unroll
-        for (int mt = 0; mt < MT; mt++) {
-            asm volatile("" : "+v"(nxt.pid[mt]));
-            if constexpr (!G::GU) asm volatile("" : "+v"(nxt.pq[mt].x), "+v"(nxt.pq[mt].y), "+v"(nxt.pq[mt].z), "+v"(nxt.pq[mt].w));
-        }
+        for (int mt = 0; mt < MT; mt++) asm volatile("" : "+v"(nxt.pid[mt]));
 #pragma unroll
-        for (int q = 0; q < NO; q++) asm volatile("" : "+v"(nxt.own[q]), "+v"(nxt.xe[q]));
+        for (int q = 0; q < NO; q++) {
+            if constexpr (G::GU) asm volatile("" : "+v"(nxt.xe[q]));
+            // this thread's output pairs are those of operand rows om % 16
+            else own[q] = __shfl(CW == 4 ? cur.pid[q] : tmt ? cur.pid[MT - 1] : cur.pid[0], om & 15);
+        }
         f32x4 acc[MT];
         for (int st = 0;; st++) {
 #pragma unroll
