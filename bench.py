@@ -120,11 +120,9 @@ def prefill_gateup_kernel(cfg) -> str:
     sgt = TYPE_NAMES[cfg.shared_types[0]] if cfg.shared_types else gt
     what = ("fp16 MFMA over Q8_0 blocks" if gt == "Q8_0" else
             f"fp16 MFMA over {gt} super-blocks, mins from activation sums")
-    # pairs per pass: 16 when the batch averages at most 10 (Q8_0) or 4 (K-quant; 16 with rows of
-    # down above 2048 columns) pairs per expert; Q2_K .. Q4_K ring slots hold two super-blocks
-    # when H allows (the library's rules)
-    wide = max(cfg.I, (cfg.shared_inter or cfg.I) if cfg.shared_types else 0) > 2048
-    m = 16 if cfg.tokens * cfg.K <= (10 if gt == "Q8_0" else 16 if wide else 4) * cfg.E else 32
+    # pairs per pass: 16 when the batch averages at most 10 pairs per expert; Q2_K .. Q4_K ring
+    # slots hold two super-blocks when H allows (the library's rules)
+    m = 16 if cfg.tokens * cfg.K <= 10 * cfg.E else 32
 
     def inst_name(t):
         two = t in ("Q2_K", "Q3_K", "Q4_K") and cfg.H % 512 == 0

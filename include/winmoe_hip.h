@@ -86,12 +86,10 @@ enum {
 #define WM_FLAG_SPIN_PROBE 16
 /* wm_layer_desc.flags, prefill only: the expert GEMMs take the batch's pairs
  * in passes of at most 16 (PASS16) or 32 (PASS32) pairs of one expert.  By
- * default a batch that averages at most 10 pairs per expert (T*K <= 10*E)
- * with Q8_0 gate/up, or at most 4 with K-quant gate/up (16 when inter or
- * inter_shared exceeds 2048), uses 16, any other 32.  The down GEMMs of a layer
- * with inter or inter_shared above 2048 always take 16, gate/up what is asked
- * for.  The results are the same bit for bit either way; only the speed
- * differs. */
+ * default a batch that averages at most 10 pairs per expert (T*K <= 10*E) uses
+ * 16, any other 32.  The down GEMMs of a layer with inter or inter_shared above
+ * 2048 always take 16, gate/up what is asked for.  The results are the same bit
+ * for bit either way; only the speed differs. */
 #define WM_FLAG_PREFILL_PASS16 32
 #define WM_FLAG_PREFILL_PASS32 64
 

@@ -136,8 +136,8 @@ def test_bench_refuses_more_than_one_gpu():
 
 def test_bench_names_the_prefill_kernels_the_library_picks():
     """The bench line's kernel names follow the library's pass-size rule (16
-    pairs up to 10 per expert for Q8_0, 4 for K-quants) and its
-    two-super-block stages for Q2_K .. Q4_K gate/up."""
+    pairs up to 10 per expert) and its two-super-block ring slots for Q2_K ..
+    Q4_K gate/up."""
     import importlib.util
     import sys
     from winmoe_amd import synth

@@ -48,22 +48,23 @@ struct PrefillArgs {
 // Pass records a prefill of T tokens may need (passes of 16 pairs or more).
 inline int64_t prefill_max_passes(int64_t T, int64_t K, int64_t E) { return (T * K + 15) / 16 + E + (T + 15) / 16 + 1; }
 
-// Pairs per pass: 16 when the batch averages at most 10 (Q8_0 gate/up) or 4
-// (K-quant gate/up) pairs per routed expert, else 32.  Passes of 16 have
-// smaller activation slots (LDS for a deeper weight ring) and a lighter
-// stage; passes of 32 stream a busy expert's rows half as often.  Measured
-// with Zipf routing over 512 experts (ms per batch, 16 / 32): Q8_0 at 10
-// pairs per expert 1.54 / 1.56, at 20 2.16 / 1.80; Q4_K gate/up, Q6_K down
-// at 3 pairs 1.45 / 1.54, at 12 2.14 / 1.95.
-// Wide rows (prefill_wide: only gate/up can take passes of 32, and the pairs
-// are grouped twice): K-quants from 16 pairs on.  us per batch, 16 / 32, 64
-// experts, I 4096: Q4_K, Q6_K, H 4096 at 6 pairs 572 / 647, at 16 769 / 762, at
-// 40 1465 / 1333; Q2_K, Q3_K, H 2048 at 12 331 / 350, at 16 363 / 360, at 28 557
-// / 508; Q8_0, H 2048 at 6 397 / 413, at 9 426 / 416, at 20 561 / 500.
+// Pairs per pass: 16 when the batch averages at most 10 pairs per routed
+// expert, else 32.  A pass of 32 streams and decodes a busy expert's rows half
+// as often and leaves its second row tile out where it is not needed, but its
+// partial sums and staging take LDS from the ring (a slot, in some instances),
+// and a small batch has fewer items to share out.  us per batch with skewed
+// routing, passes of 16 / 32, at 4, 8, 12, 16, 20 pairs per expert:
+//   Q8_0, 512 experts, H 4096, I 1024    1199/1209 1299/1271 1373/1399 1526/1418 1746/1485
+//   Q8_0, 128 experts, H 2048, I 512      106/114   128/137   130/143   138/150   160/159
+//   Q4_K, Q6_K, 512 experts, H 4096      1052/1096 1272/1280 1469/1371 1741/1579 2033/1765
+//   Q2_K, Q3_K, 128 experts, H 4096       239/257   292/296   300/328   360/362   405/397
+//   Q6_K, Q8_0, 256 experts, I 512        355/385   400/419   434/465   502/500   570/512
+// and with rows of down above 2048 columns (prefill_wide: only gate/up takes
+// passes of 32, the pairs are grouped twice), 64 experts, I 4096, at 3, 9, 12, 20, 40:
+//   Q4_K, Q6_K, H 4096    513/518 586/600 643/618 885/844 1427/1283
+//   Q8_0, H 2048          372/372 393/389 416/414 548/485  925/752
 inline bool prefill_wide(int64_t I, int64_t Is) { return I > 2048 || Is > 2048; }
-inline int prefill_pass_size(int64_t T, int64_t K, int64_t E, int gate_type, bool wide) {
-    return T * K <= (gate_type == Q8_0 ? 10 : wide ? 16 : 4) * E ? 16 : 32;
-}
+inline int prefill_pass_size(int64_t T, int64_t K, int64_t E) { return T * K <= 10 * E ? 16 : 32; }
 
 // Weight formats the expert GEMMs read: gate and up (one format for both) and down.
 inline bool prefill_type(int t) { return t == Q8_0 || t == Q2_K || t == Q3_K || t == Q4_K || t == Q5_K || t == Q6_K; }
