@@ -487,20 +487,23 @@ def test_prefill_router_kernels_agree(wm):
                                      (33, 40, 4096, 16), (360, 352, 256, 16), (545, 250, 1024, 16), (1025, 126, 256, 9)])
 def test_prefill_router_tiles(wm, orc, T, E, H, K):
     """The matrix-core router at the edges of its tiles (16 x 16 below 128
-    tiles of 32 x 32, 32 x 32 from there; H of 2 to 32 chunks of 128): picks
-    and weights are those of the plain kernel (same layer, router 4 bytes past
-    a 16-byte boundary) bit for bit, with rows of subnormal, huge and equal
-    router values among the others."""
+    tiles of 32 x 32, 32 x 32 from there; H of 2 to 32 chunks of 128): logits,
+    picks and weights are those of the plain kernel (same layer, router 4 bytes
+    past a 16-byte boundary) bit for bit, with rows of subnormal, huge, infinite
+    and equal router values and a token of tiny ones among the others."""
+    import ctypes as C
     import torch
     from winmoe_amd.moe import MoELayer
     g = torch.Generator(device="cuda")
     g.manual_seed(T * 131 + E)
     R = 0.02 * torch.randn(E, H, generator=g, device="cuda")
     R[E // 2] = R[E // 3]
-    R[0] *= 1e-37
+    R[0] *= 1e-38                                       # subnormal values, products and sums
     R[E - 1] *= 1e30
+    R[E - 2, ::7] *= 1e-38                              # normal and subnormal products in one chain
+    R[1, H // 2] = float("inf")
     X = torch.randn(T, H, generator=g, device="cuda").to(torch.bfloat16)
-    X[T // 2] *= 1e-30
+    X[T // 2] *= 3e-38                                  # its products with the ordinary rows are subnormal
     buf = torch.zeros(E * H + 4, dtype=torch.float32, device="cuda")
     shifted = buf[1:1 + E * H].view(E, H)
     shifted.copy_(R)
@@ -508,11 +511,21 @@ def test_prefill_router_tiles(wm, orc, T, E, H, K):
     W = torch.zeros(E * I * (H // 32) * 34, dtype=torch.uint8, device="cuda")
     ws = [MoELayer(H, I, E, K, r, W, W, W, (Q8_0, Q8_0, Q8_0), max_tokens=T) for r in (R, shifted)]
     case(f"prefill router tiles T={T} E={E} H={H}")
+    logits = []
     for L in ws:
         L.prefill(X)
+        off = [C.c_int64() for _ in range(3)]
+        wm.load().wm_prefill_workspace_routing(C.byref(L.desc), L.pf_tokens, *[C.byref(o) for o in off])
+        o = off[2].value - (L.pf_tokens * E * 4 + 255) // 256 * 256      # [T][E], ahead of the counters
+        logits.append(host(L.pf_ws[o:o + 4 * T * E].view(torch.float32)).reshape(T, E).copy())
+    assert same_bits_nan(*logits)
+    assert np.array_equal(logits[0][:, E // 2].view(np.uint32), logits[0][:, E // 3].view(np.uint32))
+    subnormal = lambda v: ((np.abs(v) > 0) & (np.abs(v) < 2.0 ** -126)).any()
+    assert subnormal(logits[0][T // 2, 2:E - 2]) and not np.isfinite(logits[0][:, 1]).any()
+    assert T == 1 or subnormal(logits[0][:, 0])         # (one token: the tiny one, 0 with row 0)
     (ia, wa), (ib, wb) = ([host(v) for v in L.prefill_routing(T)] for L in ws)
     assert np.array_equal(ia, ib)
-    assert np.array_equal(wa.view(np.uint32), wb.view(np.uint32))
+    assert same_bits_nan(wa, wb)
 
 
 def test_prefill_scales_and_narrow_shared(wm, orc):
