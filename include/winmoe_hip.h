@@ -242,8 +242,10 @@ int wm_moe_decode_stack(int n_layers, const wm_layer_desc* const* d, void* const
  * stream) holds wm_prefill_workspace_size(d, max_tokens) bytes, 256-byte
  * aligned.  x and out are 16-byte aligned.  Expert matrices (routed and
  * shared, each with its own formats): Q8_0 or Q2_K .. Q6_K, gate and up of
- * one format; 16-byte aligned with strides that are multiples of 16; H, I,
- * inter_shared multiples of 256; otherwise WM_EINVAL. */
+ * one format; 16-byte aligned with strides that are multiples of 16; H, I and
+ * inter_shared each 256, 512, 1024, 2048 or 4096 (matrix widths are
+ * powers of two up to 4096 in every entry point); otherwise WM_EINVAL, nothing
+ * launched. */
 int64_t wm_prefill_workspace_size(const wm_layer_desc* d, int max_tokens);
 int wm_moe_prefill(const wm_layer_desc* d, const uint16_t* x_bf16, int T, float* out, void* ws,
                    int64_t ws_bytes, int max_tokens, void* stream);

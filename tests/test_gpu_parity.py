@@ -696,7 +696,8 @@ def test_prefill_row_tiles(wm, orc, H, I, types):
 
 
 def test_prefill_rejects_unsupported_widths(wm):
-    """Prefill needs H, I and the shared width to be multiples of 256."""
+    """Prefill needs H, I and the shared width to be powers of two from 256 to
+    4096 (384: not one; the others below)."""
     from winmoe_amd import synth
     cfg = _pf_cfg(E=8, K=2, H=384, I=256)
     sl = synth.build_layer(cfg, max_tokens=4)
@@ -704,6 +705,32 @@ def test_prefill_rejects_unsupported_widths(wm):
     with pytest.raises(wm.WinMoEError) as ei:
         sl.layer.prefill(X)
     assert ei.value.rc == wm._lib.WM_EINVAL
+
+
+@pytest.mark.parametrize("H,I,Is", [(768, 256, 0), (1536, 512, 256), (5120, 256, 0), (8192, 256, 0), (256, 768, 0),
+                                    (512, 1536, 512), (256, 8192, 0), (256, 512, 768), (512, 256, 128), (128, 256, 0)])
+def test_prefill_refuses_widths_before_it_starts(wm, H, I, Is):
+    """Widths that are multiples of 256 but not powers of two up to 4096 (and
+    those below 256) are refused with WM_EINVAL before anything is launched:
+    the hit counters stay at zero."""
+    import ctypes as C
+    import torch
+    from winmoe_amd import synth
+    E, K, T = 8, 2, 4
+    cfg = synth.LayerConfig(f"pf_w_{H}_{I}_{Is}", E=E, K=K, H=H, I=I, types=(Q8_0, Q8_0, Q8_0),
+                            shared_types=(Q8_0,) * 3 if Is else None, shared_inter=Is, tokens=1, routing="zipf",
+                            x_dtype="bf16", seed=3)
+    sl = synth.build_layer(cfg, max_tokens=T)
+    X = synth.make_hidden(cfg, tokens=T)
+    ids = np.tile(np.arange(K, dtype=np.int32), (T, 1))
+    case(f"prefill refuses H={H} I={I} shared={Is}")
+    with pytest.raises(wm.WinMoEError) as ei:
+        sl.layer.prefill_forced(X, dev(ids), dev(np.full((T, K), 0.5, np.float32)))
+    assert ei.value.rc == wm._lib.WM_EINVAL
+    off = [C.c_int64() for _ in range(3)]
+    wm.load().wm_prefill_workspace_routing(C.byref(sl.layer.desc), sl.layer.pf_tokens, *[C.byref(o) for o in off])
+    o = off[2].value
+    assert not host(sl.layer.pf_ws[o:o + 4 * E].view(torch.int32)).any()
 
 
 @pytest.mark.parametrize("types", [(Q4_K, Q5_K, Q6_K), (Q8_0, Q6_K, Q8_0)])

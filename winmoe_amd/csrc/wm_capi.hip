@@ -986,10 +986,11 @@ static int run_prefill(const wm_layer_desc* d, const uint16_t* x, int T, const i
     const bool types = d->gate_type == d->up_type && prefill_type(d->gate_type) && prefill_type(d->down_type) &&
                        (!sh || (d->sh_gate_type == d->sh_up_type && prefill_type(d->sh_gate_type) &&
                                 prefill_type(d->sh_down_type)));
+    // powers of two up to 4096 (check_matrix), whole super-blocks
     const bool shapes = d->hidden % 256 == 0 && d->inter % 256 == 0 && (!sh || Ishared(d) % 256 == 0);
     if (!types || !shapes) {
         fprintf(stderr, "winmoe_hip: prefill needs quantised expert matrices (Q8_0, Q2_K .. Q6_K) with gate and up "
-                        "of one format, and H, I multiples of 256\n");
+                        "of one format, and H, I powers of two from 256 to 4096\n");
         return WM_EINVAL;
     }
     if (wm_init()) return WM_ERR;

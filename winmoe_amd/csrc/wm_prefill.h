@@ -70,8 +70,8 @@ inline int prefill_pass_size(int64_t T, int64_t K, int64_t E) { return T * K <= 
 inline bool prefill_type(int t) { return t == Q8_0 || t == Q2_K || t == Q3_K || t == Q4_K || t == Q5_K || t == Q6_K; }
 
 // The phases of a prefill, stream-ordered (the caller checks types: gate and
-// up of one format, formats the GEMMs read, H, I, Is multiples of 256, expert
-// strides multiples of 16):
+// up of one format, formats the GEMMs read, H, I, Is powers of two from 256 to
+// 4096, expert strides multiples of 16):
 //   routing: router + top-K, or the caller's ids / weights; grouping; shared
 //   gate; fp16 copy of x
 //   gate/up + SwiGLU, down projection, combine.
