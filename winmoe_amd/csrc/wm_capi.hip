@@ -927,7 +927,7 @@ extern "C" int wm_expert_ffn(const void* gate, int gt, const void* up, int ut, c
 // ------------------------------------------------------------------ prefill
 
 struct PfLayout {
-    int64_t status, ids, w, logits, hits, offsets, sorted, passes, pass_count, sg, x16, xexp, act_hi, act_lo, act_sc, y,
+    int64_t status, ids, w, logits, hits, sorted, passes, pass_count, sg, x16, xexp, act_hi, act_lo, act_sc, y,
         total;
     int64_t act_stride;
 };
@@ -944,7 +944,6 @@ static PfLayout pf_layout(const wm_layer_desc* d, int max_tokens) {
     L.w = o; o += up256(T * K * 4);
     L.logits = o; o += up256(T * E * 4);
     L.hits = o; o += up256(E * 4);
-    L.offsets = o; o += up256((E + 2) * 4);
     L.sorted = o; o += up256(pairs * 4);
     L.passes = o; o += up256(prefill_max_passes(T, K, E) * 256);
     L.pass_count = o; o += 256;
@@ -1010,7 +1009,7 @@ static int run_prefill(const wm_layer_desc* d, const uint16_t* x, int T, const i
     a.sh_gate_inp = sh ? d->sh_gate_inp : nullptr;
     a.ids = (int32_t*)(w8 + L.ids); a.w = (float*)(w8 + L.w); a.logits = (float*)(w8 + L.logits);
     a.hits = (uint32_t*)(w8 + L.hits); a.status = (int32_t*)(w8 + L.status);
-    a.offsets = (int32_t*)(w8 + L.offsets); a.sorted = (int32_t*)(w8 + L.sorted); a.sg = (float*)(w8 + L.sg);
+    a.sorted = (int32_t*)(w8 + L.sorted); a.sg = (float*)(w8 + L.sg);
     a.passes = (int32_t*)(w8 + L.passes); a.pass_count = (int32_t*)(w8 + L.pass_count);
     a.x16 = (uint16_t*)(w8 + L.x16); a.xexp = (int32_t*)(w8 + L.xexp);
     a.act_hi = (uint16_t*)(w8 + L.act_hi); a.act_lo = (uint16_t*)(w8 + L.act_lo); a.act_sc = (float*)(w8 + L.act_sc);

@@ -1043,7 +1043,7 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
 #endif
 
 // A CU holds 8 waves either way: one workgroup of 8, or two of 4.
-template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB, int CW = 8>
+template <int AHL, int WT, int M, int NSB, int CW>
 __global__ __launch_bounds__(64 * CW, 2) void k_pf_gemm(PfGemm a) {
 #if defined(__HIP_DEVICE_COMPILE__)
     const int n_rp = a.npass[0], n_r = a.sel == 2 ? 0 : n_rp * a.nrb_r;
@@ -1088,20 +1088,20 @@ template <class G> bool pf_gemm_plan(PfGemm& h, int cw) {
 // I 512 (both), Q8_0 top-4 of 64 at 1001 tokens 197 / 179.
 WM_HD inline int gm_waves(bool gateup, int ncol) { return ncol / gm_slice(gateup, ncol) <= 4 ? 4 : 8; }
 
-template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB, int CW>
+template <int AHL, int WT, int M, int NSB, int CW>
 int launch_pf_gemm_cw(PfGemm h, int n_wg, hipStream_t s) {
     typedef GmGeo<AHL, WT, M, NSB, CW> G;
     if (!pf_gemm_plan<G>(h, CW)) return (int)hipErrorInvalidValue;
-    hipError_t e = hipFuncSetAttribute((const void*)k_pf_gemm<NMAT, AHL, NSUB, WT, M, NSB, CW>,
+    hipError_t e = hipFuncSetAttribute((const void*)k_pf_gemm<AHL, WT, M, NSB, CW>,
                                        hipFuncAttributeMaxDynamicSharedMemorySize, G::LDS);
     if (e != hipSuccess) return (int)e;
-    hipLaunchKernelGGL((k_pf_gemm<NMAT, AHL, NSUB, WT, M, NSB, CW>), dim3(n_wg * (8 / CW)), dim3(64 * CW), G::LDS, s, h);
+    hipLaunchKernelGGL((k_pf_gemm<AHL, WT, M, NSB, CW>), dim3(n_wg * (8 / CW)), dim3(64 * CW), G::LDS, s, h);
     return (int)hipGetLastError();
 }
-template <int NMAT, int AHL, int NSUB, int WT, int M, int NSB = 1>
+template <int AHL, int WT, int M, int NSB = 1>
 int launch_pf_gemm(const PfGemm& g, int n_wg, hipStream_t s) {
-    if (gm_waves(AHL == 1, g.ncol) == 4) return launch_pf_gemm_cw<NMAT, AHL, NSUB, WT, M, NSB, 4>(g, n_wg, s);
-    return launch_pf_gemm_cw<NMAT, AHL, NSUB, WT, M, NSB, 8>(g, n_wg, s);
+    if (gm_waves(AHL == 1, g.ncol) == 4) return launch_pf_gemm_cw<AHL, WT, M, NSB, 4>(g, n_wg, s);
+    return launch_pf_gemm_cw<AHL, WT, M, NSB, 8>(g, n_wg, s);
 }
 
 template <int AHL, int WT, int M, int NSB, int SWT, int CW>

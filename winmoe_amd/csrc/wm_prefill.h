@@ -28,8 +28,7 @@ struct PrefillArgs {
     float* logits;              // [T][E]
     uint32_t* hits;             // [E]
     int32_t* status;
-    int32_t* offsets;           // [E + 2]: pairs of expert e are sorted[offsets[e] .. offsets[e + 1]); shared: [E] .. [E + 1]
-    int32_t* sorted;            // [T * K + T] pair indices grouped by expert
+    int32_t* sorted;            // [T * K + T] pair indices grouped by expert (batches that outgrow k_pf_group's LDS)
     int32_t* passes;            // [prefill_max_passes][64] pass records (up to pass_m pairs of one expert)
     int32_t* pass_count;        // [2]: routed passes, shared passes
     uint16_t* x16;              // fp16 [T][H]: x * 2^-e per token

@@ -15,13 +15,16 @@
 //   k_pf_group     counting sort of the pairs by expert; passes of <= 16
 //                  or 32 pairs of one expert (prefill_pass_size)
 //   k_pf_gemm      gate and up + SwiGLU on fp16 MFMA, persistent: one
-//                  workgroup per CU streams (pass, 128-row block) items
-//                  through an LDS-DMA ring; the SwiGLU output is stored as
-//                  fp16 hi + lo times a power of two per (pair, 128 rows);
-//                  then the down projection of the same form (hi and lo:
-//                  two MFMAs) (both in wm_pf_gemm.h, one instance per weight
-//                  format; routed and shared experts of different formats
-//                  take a launch each)
+//                  workgroup of 8 waves or two of 4 per CU work through
+//                  (pass, 128-row block) items, every wave streaming its
+//                  columns of the rows through an LDS-DMA ring of its own; the
+//                  SwiGLU output is stored as fp16 hi + lo times a power of
+//                  two per (pair, 128 rows); then the down projection of the
+//                  same form (hi and lo: two MFMAs) (both in wm_pf_gemm.h, one
+//                  instance per weight format)
+//   k_pf_gemm2     routed K-quant passes and a few shared Q8_0 ones in one
+//                  launch (shared experts of another format or width else
+//                  take a launch of their own)
 //   k_pf_combine   per token: sum_k w_k y_k in k order + gate * y_shared
 #include <hip/hip_runtime.h>
 #include <stdint.h>
@@ -319,10 +322,9 @@ constexpr int PG_REG = 8, PG_SORT = 45056, PG_XEXP = 8192, PG_MAP = 4096;
 // by kmul = ceil(2^32 / K) instead of a division, and ids are read PG_REG to
 // a thread at a time: 512 tokens top-10 23 -> 11 us, 4096 tokens 114 -> 27.
 __global__ __launch_bounds__(1024) void k_pf_group(const int32_t* __restrict__ ids, int T, int K, uint32_t kmul, int E,
-                                                   int has_shared, int pm, int32_t* __restrict__ offsets,
-                                                   int32_t* __restrict__ sorted, int32_t* __restrict__ passes,
-                                                   int32_t* __restrict__ pass_count, const int32_t* __restrict__ xexp,
-                                                   uint32_t* __restrict__ hits) {
+                                                   int has_shared, int pm, int32_t* __restrict__ sorted,
+                                                   int32_t* __restrict__ passes, int32_t* __restrict__ pass_count,
+                                                   const int32_t* __restrict__ xexp, uint32_t* __restrict__ hits) {
     __shared__ int cnt[1025];
     __shared__ int off[1026];
     __shared__ int pbase[1026];
@@ -376,7 +378,6 @@ __global__ __launch_bounds__(1024) void k_pf_group(const int32_t* __restrict__ i
         pbase[G] = carry.y;
     }
     __syncthreads();
-    for (int e = tid; e <= G; e += 1024) offsets[e] = off[e];
     if (tid == 0) {
         pass_count[0] = pbase[E];
         pass_count[1] = pbase[G] - pbase[E];
@@ -565,8 +566,8 @@ __global__ __launch_bounds__(256) void k_pf_combine(PrefillArgs a) {
 
 static void launch_group(const PrefillArgs& a, uint32_t* hits, hipStream_t s) {
     const uint32_t kmul = (uint32_t)(((1ull << 32) + a.K - 1) / a.K);       // (0 for K = 1)
-    hipLaunchKernelGGL(k_pf_group, dim3(1), dim3(1024), 0, s, a.ids, a.T, a.K, kmul, a.E, a.has_shared, a.pass_m, a.offsets,
-                       a.sorted, a.passes, a.pass_count, a.xexp, hits);
+    hipLaunchKernelGGL(k_pf_group, dim3(1), dim3(1024), 0, s, a.ids, a.T, a.K, kmul, a.E, a.has_shared, a.pass_m, a.sorted,
+                       a.passes, a.pass_count, a.xexp, hits);
 }
 
 int launch_prefill_route(const PrefillArgs& a, const int32_t* forced_ids, const float* forced_w, hipStream_t s) {
@@ -593,7 +594,7 @@ int launch_prefill_route(const PrefillArgs& a, const int32_t* forced_ids, const 
 // One gate/up or down GEMM launch of format wt over the passes sel selects,
 // for passes of m pairs.
 template <int M> static int launch_q8(bool gateup, const PfGemm& g, int n_wg, hipStream_t s) {
-    return gateup ? launch_pf_gemm<1, 1, 2, Q8_0, M>(g, n_wg, s) : launch_pf_gemm<1, 2, 1, Q8_0, M>(g, n_wg, s);
+    return gateup ? launch_pf_gemm<1, Q8_0, M>(g, n_wg, s) : launch_pf_gemm<2, Q8_0, M>(g, n_wg, s);
 }
 static int launch_fmt(int m, bool gateup, int wt, const PfGemm& g, int n_wg, hipStream_t s) {
     if (wt != Q8_0) return launch_pf_gemm_kq(m, gateup, wt, g, n_wg, s);

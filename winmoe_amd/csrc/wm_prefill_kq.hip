@@ -12,7 +12,7 @@ template <int AHL, int WT, int M, int NSB> static int go(const PfGemm& g, const 
     if constexpr (AHL == 1 || M == 16)
         if (sh) return launch_pf_gemm2<AHL, WT, M, NSB, Q8_0>(g, *sh, n_wg, s);
     if (sh) return (int)hipErrorInvalidValue;
-    return launch_pf_gemm<1, AHL, AHL == 1 ? 2 : 1, WT, M, NSB>(g, n_wg, s);
+    return launch_pf_gemm<AHL, WT, M, NSB>(g, n_wg, s);
 }
 
 // Gate/up: ring slots of two super-blocks (512 columns) for the formats whose
