@@ -113,42 +113,67 @@ def prefill_gateup_bytes(cfg, ids) -> int:
     return b
 
 
-def prefill_gateup_kernel(cfg) -> str:
-    """What the prefill gate/up phase launches for the workload's formats."""
+def prefill_gateup_instances(cfg):
+    """Template arguments (format names for the formats) of the kernels that the
+    prefill gate/up phase launches for the workload, by the library's rules."""
     from winmoe_amd import TYPE_NAMES
     gt = TYPE_NAMES[cfg.types[0]]
     sgt = TYPE_NAMES[cfg.shared_types[0]] if cfg.shared_types else gt
-    what = ("fp16 MFMA over Q8_0 blocks" if gt == "Q8_0" else
-            f"fp16 MFMA over {gt} super-blocks, mins from activation sums")
     # pairs per pass: 16 when the batch averages at most 10 pairs per expert; Q2_K .. Q4_K ring
-    # slots hold two super-blocks when H allows (the library's rules)
+    # slots hold two super-blocks when H allows; workgroups of 4 waves up to 4 slices of 512 columns
     m = 16 if cfg.tokens * cfg.K <= 10 * cfg.E else 32
+    waves = 4 if cfg.H <= 2048 else 8
 
-    def inst_name(t):
-        two = t in ("Q2_K", "Q3_K", "Q4_K") and cfg.H % 512 == 0
-        return f"k_pf_gemm<1,1,2,{t},{m},{2 if two else 1}>"
-    inst = {t: inst_name(t) for t in (gt, sgt)}
+    def blocks(t):
+        return 2 if t in ("Q2_K", "Q3_K", "Q4_K") and cfg.H % 512 == 0 else 1
     if sgt == gt:
-        return f"{inst[gt]} (prefill gate+up+SwiGLU: {what}, LDS-DMA ring)"
-    return (f"{inst[gt]} + {inst[sgt]} (prefill gate+up+SwiGLU phase: routed {gt} "
-            f"launch and shared-expert {sgt} launch; {what})")
+        return [("k_pf_gemm", 1, gt, m, blocks(gt), waves)]
+    # a few Q8_0 shared passes ride in the routed K-quants' launch: less than half a round of the grid
+    items = (cfg.tokens + m - 1) // m * ((cfg.shared_inter or cfg.I) // 128)
+    if gt != "Q8_0" and sgt == "Q8_0" and 2 * items < 256 * (8 // waves):
+        return [("k_pf_gemm2", 1, gt, m, blocks(gt), sgt, waves)]
+    return [("k_pf_gemm", 1, t, m, blocks(t), waves) for t in (gt, sgt)]
 
 
-def committed_traffic(kernel, workload):
+def prefill_gateup_kernel(cfg) -> str:
+    """What the prefill gate/up phase launches for the workload's formats."""
+    inst = prefill_gateup_instances(cfg)
+    gt = inst[0][2]
+    what = ("fp16 MFMA over Q8_0 blocks" if gt == "Q8_0" else
+            f"fp16 MFMA over {gt} super-blocks, mins in a second MFMA")
+    names = [f"{i[0]}<{','.join(str(v) for v in i[1:])}>" for i in inst]
+    if len(inst) == 1:
+        return f"{names[0]} (prefill gate+up+SwiGLU: {what}, LDS-DMA rings)"
+    return (f"{' + '.join(names)} (prefill gate+up+SwiGLU phase: routed {gt} "
+            f"launch and shared-expert {inst[1][2]} launch; {what})")
+
+
+def kernel_signatures(inst):
+    """The instances as rocprofv3 names them (format numbers)."""
+    from winmoe_amd import TYPE_NAMES
+    num = {n: t for t, n in TYPE_NAMES.items()}
+    return [f"{i[0]}<{', '.join(str(num.get(v, v)) for v in i[1:])}>" for i in inst]
+
+
+def committed_traffic(kernel, workload, signatures=()):
     """HBM bytes per launch of `kernel` on `workload` from the committed
-    rocprofv3 PMC summary (FETCH_SIZE + WRITE_SIZE, calibrated), or None."""
+    rocprofv3 PMC summary (FETCH_SIZE + WRITE_SIZE, calibrated), or None; None
+    too when the summary counted other instances than `signatures`."""
     path = os.path.join(ROOT, "profiles", f"{kernel}_{workload}_traffic.json")
     try:
         with open(path) as f:
-            return json.load(f).get("traffic_bytes_per_launch")
+            prof = json.load(f)
     except (OSError, ValueError):
         return None
+    if any(s not in prof.get("kernel", "") for s in signatures):
+        return None
+    return prof.get("traffic_bytes_per_launch")
 
 
-def roofline(kernel_desc, kernel, workload, per_launch, launch_us):
+def roofline(kernel_desc, kernel, workload, per_launch, launch_us, signatures=()):
     ach = per_launch / (launch_us * 1e-6) / 1e9
     return {"bound": "hbm", "achieved": round(ach, 1), "peak": PEAK_HBM_GBPS, "unit": "GB/s",
-            "frac": round(ach / PEAK_HBM_GBPS, 4), "traffic": committed_traffic(kernel, workload),
+            "frac": round(ach / PEAK_HBM_GBPS, 4), "traffic": committed_traffic(kernel, workload, signatures),
             "kernel": kernel_desc, "bytes_per_launch": per_launch, "avg_launch_us": round(launch_us, 2)}
 
 
@@ -320,7 +345,7 @@ def entry(wl, L, steps, warmup, multi_kernel=False):
     if wl.prefill and "gate_up_swiglu" in phases:
         gu = phases["gate_up_swiglu"]
         rl = roofline(prefill_gateup_kernel(cfg), "k_pf_gemm", cfg.name, prefill_gateup_bytes(cfg, wl.route_ids(0)),
-                      gu["avg_us"])
+                      gu["avg_us"], kernel_signatures(prefill_gateup_instances(cfg)))
     elif wl.stack:
         # one chained launch per token moves all the layers' bytes
         launch_us = 1000.0 * ev_ms / steps

@@ -136,8 +136,11 @@ def test_bench_refuses_more_than_one_gpu():
 
 def test_bench_names_the_prefill_kernels_the_library_picks():
     """The bench line's kernel names follow the library's pass-size rule (16
-    pairs up to 10 per expert) and its two-super-block ring slots for Q2_K ..
-    Q4_K gate/up."""
+    pairs up to 10 per expert), its two-super-block ring slots for Q2_K .. Q4_K
+    gate/up, its workgroups (8 waves for H 4096, 4 for H 2048) and its merged
+    launch of a few shared passes; a traffic summary that counted other
+    instances is not quoted."""
+    import dataclasses
     import importlib.util
     import sys
     from winmoe_amd import synth
@@ -146,6 +149,13 @@ def test_bench_names_the_prefill_kernels_the_library_picks():
     bench = importlib.util.module_from_spec(spec)
     sys.modules["bench_mod"] = bench
     spec.loader.exec_module(bench)
-    assert bench.prefill_gateup_kernel(synth.CONFIGS["c5"]).startswith("k_pf_gemm<1,1,2,Q8_0,16,1>")
-    c3p = bench.prefill_gateup_kernel(synth.CONFIGS["c3p"])
-    assert c3p.startswith("k_pf_gemm<1,1,2,Q4_K,16,2> + k_pf_gemm<1,1,2,Q8_0,16,1>")
+    c5, c3p = synth.CONFIGS["c5"], synth.CONFIGS["c3p"]
+    name = bench.prefill_gateup_kernel
+    assert name(c5).startswith("k_pf_gemm<1,Q8_0,16,1,8>")
+    assert name(c3p).startswith("k_pf_gemm<1,Q4_K,16,2,8> + k_pf_gemm<1,Q8_0,16,1,8>")
+    assert name(dataclasses.replace(c3p, tokens=23)).startswith("k_pf_gemm2<1,Q4_K,16,2,Q8_0,8>")
+    assert name(dataclasses.replace(c5, tokens=513, H=2048)).startswith("k_pf_gemm<1,Q8_0,32,1,4>")
+    sig = bench.kernel_signatures(bench.prefill_gateup_instances(c3p))
+    assert sig == ["k_pf_gemm<1, 12, 16, 2, 8>", "k_pf_gemm<1, 8, 16, 1, 8>"]
+    assert bench.committed_traffic("k_pf_gemm", c3p.name, ["k_pf_gemm<1, 12, 32, 2, 8>"]) is None
+    assert bench.committed_traffic("k_pf_gemm", "no such workload") is None
