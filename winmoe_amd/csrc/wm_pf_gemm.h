@@ -194,12 +194,14 @@ WM_HD int pf_item_slot(int b, int grid, int R) {
 }
 
 // With passes of 32 pairs (busy experts of several passes), in a round that
-// every workgroup has an item of, an XCD takes a contiguous run of them: the
-// passes of an expert then read its rows from that XCD's L2.  4096 tokens
-// top-10, Q8_0 (80 pairs per expert): 3631 -> 3541 us per batch, 1001 tokens,
-// 64 experts 182.5 -> 179.1.  Passes of 16 keep the spread order (512 tokens
-// Q8_0 1374, in runs 1377; Q4_K 940, 936), as does the last, partial round
-// (1001 tokens in runs there too: 205).
+// every workgroup has an item of, an XCD takes a contiguous run of them: some
+// of the passes of an expert then find its rows in that XCD's L2.  4096 tokens
+// top-10, Q8_0 (about 3 passes per expert): L2 misses of gate/up 2.53 times the
+// matrices, 3.09 without the runs, of down 2.23 and 3.03; 3631 -> 3541 us per
+// batch.  1001 tokens, 64 experts: 1.50 and 2.54 times, 182.5 -> 179.1 us.
+// Passes of 16 keep the spread order (512 tokens Q8_0 1374, in runs 1377; Q4_K
+// 940, 936), as does the last, partial round (1001 tokens in runs there too:
+// 205).
 WM_HD int pf_item_slot_full(int b, int grid) {
     return grid % PF_XCDS ? b : (b % PF_XCDS) * (grid / PF_XCDS) + b / PF_XCDS;
 }
@@ -766,7 +768,9 @@ WM_DEV void pf_gemm_items(const PfGemm& a, int n_rp, int n_r, int n_items, int l
         }
     };
     // the current pass fills its second row tile: a pass of 32 with 16 pairs or
-    // fewer leaves that tile's loads, products and sums out
+    // fewer leaves that tile's loads, products and sums out (2000 tokens Q4_K,
+    // about 12 pairs per expert: 1653 -> 1455 us per batch; a launch whose passes
+    // are all full pays up to 4 % for the branch)
     bool two = false;
     // K-quant operands hold their 8 columns in the order 0 2 1 3 4 6 5 7
     auto order_act = [&]() __attribute__((always_inline)) {
@@ -1057,7 +1061,7 @@ __global__ __launch_bounds__(64 * CW, 2) void k_pf_gemm(PfGemm a) {
 // workgroups without an item of the last round take them.  A launch of their
 // own left most of the chip idle at both ends: 2 passes of gate/up are 16
 // items, 38 us.  23 tokens through 512 experts of H 4096, I 1024, Q4_K, Q6_K,
-// top-3, Q8_0 shared: 238 us per batch with two launches, 195 with one (the
+// top-3, Q8_0 shared: 231 us per batch with two launches, 208 with one (the
 // same bits).
 template <int AHL, int WT, int M, int NSB, int SWT, int CW>
 __global__ __launch_bounds__(64 * CW, 2) void k_pf_gemm2(PfGemm r, PfGemm s) {
@@ -1083,9 +1087,10 @@ template <class G> bool pf_gemm_plan(PfGemm& h, int cw) {
 // and those of the two workgroups do not wait for each other: one computes
 // while the other is at its barrier or waits for its partial sums.  us per
 // batch with one workgroup of 8 / two of 4 (the same bits): H 4096, I 1024
-// (down alone), Q8_0 top-10 at 512 tokens 1326 / 1312, at 4096 tokens 4018 /
-// 3719; Q4_K, Q6_K top-3 at 512 tokens 995 / 950, at 2000 1656 / 1582; H 2048,
-// I 512 (both), Q8_0 top-4 of 64 at 1001 tokens 197 / 179.
+// (down alone), Q8_0 top-10 at 512 tokens 1404 / 1399, at 4096 tokens 3988 /
+// 3639; Q4_K, Q6_K top-3 at 512 tokens 993 / 959, at 2000 1473 / 1425; H 2048,
+// I 512 (both), Q8_0 top-4 of 64 at 1001 tokens 201 / 174 (at 8 tokens, where
+// few items are left to share, 63 / 69).
 WM_HD inline int gm_waves(bool gateup, int ncol) { return ncol / gm_slice(gateup, ncol) <= 4 ? 4 : 8; }
 
 template <int AHL, int WT, int M, int NSB, int CW>

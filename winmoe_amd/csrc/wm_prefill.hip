@@ -619,8 +619,8 @@ static int launch_split(int m, bool gateup, PfShape r, PfShape sh, bool has_shar
     h.rb = (int32_t)matrix_bytes(sh.wt, 1, sh.ncol);
     // One launch when the shared items are less than half a round of the
     // workgroups; from there a launch of their own fills the chip, and the two
-    // kernels keep their registers (512 tokens: 977 us per batch against 992,
-    // 2000: 1651 / 1663).
+    // kernels keep their registers (two launches / one, us per batch: 23 tokens
+    // 231 / 208, 512 tokens 952 / 965, 2000 tokens level).
     const int grid = n_wg * (8 / gm_waves(gateup, r.ncol)), items = (g.T + m - 1) / m * g.nrb_s;
     if (r.wt != Q8_0 && sh.wt == Q8_0 && (gateup || m == 16) && 2 * items < grid)
         return launch_pf_gemm_kq_q8(m, gateup, r.wt, g, h, n_wg, s);
@@ -647,9 +647,10 @@ int launch_prefill_gateup(const PrefillArgs& a, hipStream_t s) {
 // whose items are then fewer than two rounds of the workgroups (two per CU)
 // takes 256, and 128 below half a round, so that the rounds come out even.
 // us per batch, 512 / 256 / 128 rows: 8 tokens, 64 experts, H 2048 (0.3
-// rounds) 75 / 61 / 57; 1001 tokens, 64 experts, H 2048 (1.5) 179 / 177 /
-// 195; 300 tokens, 128 experts, H 2048 (1.6) 165 / 158 / 166; 90 tokens, 256
-// experts, H 4096 (3.5) 222 / 231 / 238; 4096 tokens Q8_0 3719 / 3841 / 4245.
+// rounds) 77 / 70 / 69; 1001 tokens, 64 experts, H 2048 (1.5) 179 / 174 /
+// 190; 300 tokens, 128 experts, H 2048 (1.6) 159 / 153 / 153; 512 tokens Q4_K,
+// Q6_K, 512 experts, H 4096 (10) 956 / 966 / 983; 4096 tokens Q8_0 3627 / 3781
+// / 4112.
 static int down_rows(const PrefillArgs& a) {
     const int64_t pairs = (int64_t)a.T * a.K, m = a.pass_m;
     const int64_t passes = std::min<int64_t>(pairs, a.E) + pairs / m + (a.has_shared ? a.T / m : 0);
